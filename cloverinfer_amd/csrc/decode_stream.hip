@@ -405,7 +405,8 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
   }
 }
 
-// One wave per (sequence, query head).
+// NW waves per (sequence, query head): one, four rows to a workgroup, or
+// kMergeWaves, one row to a workgroup (launch_sreduce_t chooses).
 // NEW: the partials cover context_lens[s] tokens and the merge takes
 // sequence s's new token as one more row: score q[s, h] . key_new[s, kvh]
 // in the scale of the partials (fp32 products of the 16-bit values, as the
@@ -413,10 +414,12 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
 // kv head's first query head also writes the token's key and value rows at
 // slot_mapping[s] (skipped when negative or past the pools), for the decode
 // steps after this one.
-template <typename T, int D, bool NEW = false>
-__global__ void __launch_bounds__(256) stream_reduce(const DecodeParams p) {
+template <typename T, int D, bool NEW, int NW>
+__global__ void __launch_bounds__(NW > 1 ? NW * 64 : 256) stream_reduce(const DecodeParams p) {
   constexpr int EPL = (D + 63) / 64;
-  const int64_t idx = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  __shared__ float smem[NW > 1 ? NW * (D + 1) : 1];
+  const int64_t idx = NW > 1 ? (int64_t)blockIdx.x
+                             : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (idx >= (int64_t)p.num_seqs * p.num_heads) return;
   const int s = (int)(idx / p.num_heads);
   const int h = (int)(idx - (int64_t)s * p.num_heads);
@@ -473,8 +476,8 @@ __global__ void __launch_bounds__(256) stream_reduce(const DecodeParams p) {
   const int64_t row0 = (n > 0 ? (((int64_t)seg + w0) * HG + wk) * 16 : 0) + g;
   T *dst = (T *)p.out + (int64_t)s * p.out_stride_seq + (int64_t)h * p.out_stride_head;
   if constexpr (!NEW) {
-    lse_merge<T, D, 1>(p.ws_m + row0, p.ws_l + row0, p.ws_o + row0 * D, 16 * HG, 16 * HG * D, n,
-                       dst, nullptr);
+    lse_merge<T, D, NW>(p.ws_m + row0, p.ws_l + row0, p.ws_o + row0 * D, 16 * HG, 16 * HG * D, n,
+                        dst, smem);
   } else {
     // The new token as one more row: its score q . key_new in the scale of
     // the partials (log2-domain scores times ln 2), fp32 products of the
@@ -486,12 +489,13 @@ __global__ void __launch_bounds__(256) stream_reduce(const DecodeParams p) {
       xdot += in ? to_f32(qx[e]) * to_f32(kx[e]) : 0.f;
       xv[e] = in ? to_f32(vx[e]) : 0.f;
     }
-    lse_merge<T, D, 1, true>(p.ws_m + row0, p.ws_l + row0, p.ws_o + row0 * D, 16 * HG,
-                             16 * HG * D, n, dst, nullptr, xdot, p.scale_log2 * kLn2, xv);
+    lse_merge<T, D, NW, true>(p.ws_m + row0, p.ws_l + row0, p.ws_o + row0 * D, 16 * HG,
+                              16 * HG * D, n, dst, smem, xdot, p.scale_log2 * kLn2, xv);
     // The kv head's first query head writes the token's rows at its slot,
     // for the decode steps after this one (after the merge: no load of this
     // kernel waits behind these stores).
-    if (gall == 0 && slot >= 0 && slot < ((int64_t)p.num_blocks << p.block_shift)) {
+    if ((NW == 1 || threadIdx.x < 64) && gall == 0 && slot >= 0 &&
+        slot < ((int64_t)p.num_blocks << p.block_shift)) {
       const int64_t o = (slot >> p.block_shift) * p.kv_stride_block +
                         (slot & ((1 << p.block_shift) - 1)) * p.kv_stride_token +
                         (int64_t)kvh * p.kv_stride_head;
@@ -566,17 +570,36 @@ hipError_t launch_stream_t(const DecodeParams &p, hipStream_t stream) {
   return hipErrorInvalidValue;
 }
 
-template <typename T, bool NEW = false>
-hipError_t launch_sreduce_t(const DecodeParams &p, hipStream_t stream) {
+template <typename T, bool NEW, int NW>
+hipError_t launch_sreduce_tn(const DecodeParams &p, hipStream_t stream) {
   const int64_t rows = (int64_t)p.num_seqs * p.num_heads;
-  const dim3 grid((unsigned)((rows + 3) / 4));
+  const dim3 grid((unsigned)(NW > 1 ? rows : (rows + 3) / 4)), block(NW > 1 ? NW * 64 : 256);
   if (p.head_dim == 128)
-    hipLaunchKernelGGL((stream_reduce<T, 128, NEW>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((stream_reduce<T, 128, NEW, NW>), grid, block, 0, stream, p);
   else if (p.head_dim == 64)
-    hipLaunchKernelGGL((stream_reduce<T, 64, NEW>), grid, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((stream_reduce<T, 64, NEW, NW>), grid, block, 0, stream, p);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+// Waves per merged row. The groups' partials spread over the segments, so a
+// small batch leaves each row many: 4 sequences of 150..3900 tokens (28/4
+// heads) split over 256 groups, 64 partials a segment on average and over 100
+// in the longest. One wave reads them eight at a time, one memory latency per
+// round; kMergeWaves waves read 128 at a time (that call: merge 12.8 us, call
+// 22.4 -> 15.5 us). The line lies at kWideMergePartials per segment on
+// average: there (16 sequences of 255..4095 tokens, fp32) both forms take
+// 33.4 us a call, and below it one wave is done in a round or two.
+constexpr int kMergeWaves = 8;
+constexpr int kWideMergePartials = 16;
+
+template <typename T, bool NEW = false>
+hipError_t launch_sreduce_t(const DecodeParams &p, hipStream_t stream) {
+  const int64_t groups = p.num_waves / p.head_group;
+  if (groups > (int64_t)kWideMergePartials * p.num_segments)
+    return launch_sreduce_tn<T, NEW, kMergeWaves>(p, stream);
+  return launch_sreduce_tn<T, NEW, 1>(p, stream);
 }
 
 }  // namespace
