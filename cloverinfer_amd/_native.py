@@ -175,6 +175,9 @@ SIGNATURES = {
     "clv_default_num_waves": (_c_i32, []),
     "clv_default_num_waves_fp8": (_c_i32, []),
     "clv_chunked_prefill": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), _c_ptr]),
+    "clv_chunked_prefill_split": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), _c_ptr,
+                                                 ctypes.c_size_t, _c_ptr]),
+    "clv_prefill_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
 }
 
 _lock = threading.Lock()

@@ -41,6 +41,7 @@ SOURCES = [
     "decode.hip",
     "decode_stream.hip",
     "prefill.hip",
+    "prefill_f32.hip",
     "prefill_mfma.hip",
 ]
 

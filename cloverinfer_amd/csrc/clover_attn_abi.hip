@@ -9,6 +9,7 @@
 #include <stddef.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -663,7 +664,13 @@ int clv_paged_decode_fp8_partials(const clv_decode_args *a, const float *k_scale
              : CLV_ELAUNCH;
 }
 
-int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
+}  // extern "C"
+
+namespace {
+
+// Validates a prefill argument block and fills the kernel parameters.
+// num_seqs or num_tokens of 0 (nothing to do) leaves the rest unchecked.
+int fill_prefill(const clv_prefill_args *a, clv::PrefillParams *out) {
   if (a == nullptr) return CLV_EINVAL;
   if (a->dtype != CLV_F32 && a->dtype != CLV_F16 && a->dtype != CLV_BF16) return CLV_EINVAL;
   if (a->num_seqs < 0 || a->num_tokens < 0 || a->num_heads <= 0 || a->num_kv_heads <= 0 ||
@@ -674,6 +681,10 @@ int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
   if (!supported_head_dim(a->head_dim)) return CLV_EUNSUPPORTED;
   if (!isfinite(a->scale)) return CLV_EINVAL;
   if (a->num_seqs > 65535) return CLV_EUNSUPPORTED;
+  clv::PrefillParams &p = *out;
+  p = clv::PrefillParams{};
+  p.num_seqs = a->num_seqs;
+  p.num_tokens = a->num_tokens;
   if (a->num_seqs == 0 || a->num_tokens == 0) return CLV_OK;
   const int eb = elem_bytes(a->dtype);
   if (!a->out || !a->q || !a->k_cache || !a->v_cache || !a->context_lens || !a->query_start_loc)
@@ -686,7 +697,6 @@ int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
       !stride16(a->kv_stride_block, eb) || !stride16(a->kv_stride_token, eb) ||
       !stride16(a->kv_stride_head, eb))
     return CLV_EINVAL;
-  clv::PrefillParams p{};
   p.out = a->out;
   p.q = a->q;
   p.k_cache = a->k_cache;
@@ -701,8 +711,6 @@ int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
   p.kv_stride_block = a->kv_stride_block;
   p.kv_stride_token = a->kv_stride_token;
   p.kv_stride_head = a->kv_stride_head;
-  p.num_seqs = a->num_seqs;
-  p.num_tokens = a->num_tokens;
   p.num_heads = a->num_heads;
   p.num_kv_heads = a->num_kv_heads;
   p.head_dim = a->head_dim;
@@ -713,13 +721,113 @@ int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
   p.num_blocks = a->num_blocks;
   p.scale_log2 = a->scale * 1.4426950408889634f;
   p.cus_per_xcd = device_compute_units() / 8;
-  const DType dt = (DType)a->dtype;
-  hipError_t err;
-  if (clv::prefill_mfma_supported(dt, a->head_dim, a->block_size))
-    err = clv::launch_prefill_mfma(p, dt, (hipStream_t)stream);
-  else
-    err = clv::launch_prefill_valu(p, dt, (hipStream_t)stream);
+  return CLV_OK;
+}
+
+// The kernel form of a validated prefill.
+enum class PrefillKernel { kValu, kMfma, kF32 };
+
+PrefillKernel prefill_kernel(const clv::PrefillParams &p, DType dt, int block_size) {
+  if (dt == DType::F32)
+    return clv::prefill_f32_supported(p, block_size) ? PrefillKernel::kF32 : PrefillKernel::kValu;
+  return clv::prefill_mfma_supported(dt, p.head_dim, block_size) ? PrefillKernel::kMfma
+                                                                 : PrefillKernel::kValu;
+}
+
+clv::PrefillSplitShape split_shape(const clv::PrefillParams &p, PrefillKernel k) {
+  switch (k) {
+    case PrefillKernel::kF32: return clv::prefill_f32_split_shape(p);
+    case PrefillKernel::kMfma: return clv::prefill_mfma_split_shape(p);
+    default: return {0, 0};
+  }
+}
+
+size_t split_bytes(const clv::PrefillParams &p, const clv::PrefillSplitShape &sh) {
+  const size_t rows = 2 * (size_t)sh.groups * (size_t)sh.rows;
+  return round256((size_t)sh.groups * 16) + 2 * round256(rows * 4) +
+         round256(rows * (size_t)p.head_dim * 4);
+}
+
+int launch_prefill(const clv::PrefillParams &p, DType dt, PrefillKernel k,
+                   const clv::PrefillSplit *sp, hipStream_t stream) {
+  hipError_t err = hipErrorInvalidValue;
+  switch (k) {
+    case PrefillKernel::kF32: err = clv::launch_prefill_f32(p, sp, stream); break;
+    case PrefillKernel::kMfma: err = clv::launch_prefill_mfma(p, dt, sp, stream); break;
+    case PrefillKernel::kValu: err = clv::launch_prefill_valu(p, dt, stream); break;
+  }
   return err == hipSuccess ? CLV_OK : CLV_ELAUNCH;
+}
+
+}  // namespace
+
+namespace clv {
+
+PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
+                                      int tile_units, int min_tiles, bool even_rounds) {
+  const PrefillSplitShape none = {rows, 0};
+  const int64_t bq = rows / p.group;
+  const int64_t n_q = std::max<int64_t>(1, ceil_div(p.max_query_len, bq));
+  const int64_t max_tiles = ceil_div((int64_t)p.max_blocks_per_seq << p.block_shift, bk);
+  // The table width bounds every context: up to min_tiles tiles the longest
+  // item is short, and the split would cost its merge launch.
+  if (max_tiles <= min_tiles || p.cus_per_xcd <= 0) return none;
+  const int64_t entries = (int64_t)p.num_seqs * n_q;
+  if (entries > kPrefillSplitItems) return none;
+  // Units are 32-bit on the device (at most four of an item's own).
+  if (entries * p.num_kv_heads * (max_tiles + 4) * tile_units >= (int64_t)1 << 30) return none;
+  // Chunks of one length that fill whole rounds of the device: the 16-bit
+  // kernel's natural order (dispatch_slot) makes them even already.
+  const int groups = per_cu * p.cus_per_xcd * 8;
+  if (even_rounds && (int64_t)p.num_tokens == (int64_t)p.num_seqs * p.max_query_len &&
+      entries * p.num_kv_heads % groups == 0)
+    return none;
+  return {rows, groups};
+}
+
+}  // namespace clv
+
+extern "C" {
+
+int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {
+  clv::PrefillParams p;
+  const int st = fill_prefill(a, &p);
+  if (st != CLV_OK || p.num_seqs == 0 || p.num_tokens == 0) return st;
+  const DType dt = (DType)a->dtype;
+  return launch_prefill(p, dt, prefill_kernel(p, dt, a->block_size), nullptr, (hipStream_t)stream);
+}
+
+size_t clv_prefill_workspace_bytes(const clv_prefill_args *a) {
+  clv::PrefillParams p;
+  if (fill_prefill(a, &p) != CLV_OK || p.num_seqs == 0 || p.num_tokens == 0) return 0;
+  const clv::PrefillSplitShape sh = split_shape(p, prefill_kernel(p, (DType)a->dtype, a->block_size));
+  return sh.groups > 0 ? split_bytes(p, sh) : 0;
+}
+
+int clv_chunked_prefill_split(const clv_prefill_args *a, void *workspace, size_t workspace_bytes,
+                              clv_stream_t stream) {
+  clv::PrefillParams p;
+  const int st = fill_prefill(a, &p);
+  if (st != CLV_OK || p.num_seqs == 0 || p.num_tokens == 0) return st;
+  const DType dt = (DType)a->dtype;
+  const PrefillKernel k = prefill_kernel(p, dt, a->block_size);
+  const clv::PrefillSplitShape sh = split_shape(p, k);
+  if (sh.groups == 0) return launch_prefill(p, dt, k, nullptr, (hipStream_t)stream);
+  if (workspace == nullptr || workspace_bytes < split_bytes(p, sh) ||
+      ((uintptr_t)workspace & 255u) != 0)
+    return CLV_EWORKSPACE;
+  const size_t rows = 2 * (size_t)sh.groups * (size_t)sh.rows;
+  char *ws = (char *)workspace;
+  clv::PrefillSplit sp;
+  sp.groups = sh.groups;
+  sp.desc = (int32_t *)ws;
+  ws += round256((size_t)sh.groups * 16);
+  sp.ws_m = (float *)ws;
+  ws += round256(rows * 4);
+  sp.ws_l = (float *)ws;
+  ws += round256(rows * 4);
+  sp.ws_o = (float *)ws;
+  return launch_prefill(p, dt, k, &sp, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -104,6 +104,33 @@ struct PrefillParams {
   int32_t cus_per_xcd;
 };
 
+// Workspace of a split prefill (prefill_split.h): one descriptor per group
+// and two partials of `rows` rows each.
+struct PrefillSplit {
+  float *ws_o;    // [2 * groups, rows, head_dim] unnormalised contexts
+  float *ws_m;    // [2 * groups, rows] row max of the unscaled scores
+  float *ws_l;    // [2 * groups, rows] row sum
+  int32_t *desc;  // [groups, 4]
+  int32_t groups;
+};
+
+// The one argument of the MFMA prefill kernels.
+struct PrefillArgs {
+  PrefillParams p;
+  PrefillSplit sp;         // split form only
+  int32_t bq, n_qtiles;    // tokens per query tile, query tiles per sequence
+  int32_t total;           // items (one workgroup per item)
+};
+
+// Most (sequence, query tile) pairs a split prefill keeps in LDS.
+constexpr int kPrefillSplitItems = 1024;
+
+// How a prefill kernel would split a call: its rows per workgroup and the
+// number of groups (0: one workgroup per item, no workspace).
+struct PrefillSplitShape {
+  int32_t rows, groups;
+};
+
 enum class DType : int { F32 = 0, F16 = 1, BF16 = 2 };
 
 // Launchers return hipSuccess or the launch error. Shapes are pre-validated.
@@ -119,7 +146,6 @@ hipError_t launch_stream_reduce(const DecodeParams &p, DType dt, hipStream_t str
 // stream_reduce over partials of context_lens[s] tokens plus sequence s's new
 // token (key_new/value_new[s]), which it also writes at slot_mapping[s].
 hipError_t launch_stream_reduce_append(const DecodeParams &p, DType dt, hipStream_t stream);
-hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, hipStream_t stream);
 // Writes key_new/value_new[s] at position context_lens[s] - 1 of every
 // sequence (slot from its block table), for the decode shapes whose stream
 // kernel does not append itself.
@@ -128,6 +154,20 @@ hipError_t launch_append_by_table(const DecodeParams &p, int elem_bytes, hipStre
 // rounded to nearest even; key/value in CacheParams' elem_bytes (2 or 4).
 hipError_t launch_reshape_and_cache_fp8(const CacheParams &p, int src_dtype, const float *k_scales,
                                         const float *v_scales, hipStream_t stream);
+// fp16/bf16 prefill on MFMA, and fp32 prefill on MFMA; sp: the split's workspace, or null for one workgroup
+// per item.
+PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &p);
+hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *sp,
+                               hipStream_t stream);
+bool prefill_f32_supported(const PrefillParams &p, int block_size);
+PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p);
+hipError_t launch_prefill_f32(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream);
+// The decision behind the split shapes: `rows` query rows per workgroup, `bk`
+// K/V tokens per tile, `per_cu` workgroups per compute unit, at most
+// `tile_units` units per tile; no split up to `min_tiles` tiles, nor (with
+// `even_rounds`) of equal chunks that fill whole rounds of the device.
+PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
+                                      int tile_units, int min_tiles, bool even_rounds);
 hipError_t launch_prefill_valu(const PrefillParams &p, DType dt, hipStream_t stream);
 
 // Whether the MFMA decode kernel covers this shape/dtype.

@@ -1,0 +1,443 @@
+// prefill_f32.hip - chunked prefill over paged KV with fp32 MFMAs.
+//
+// Semantics as in prefill.hip: query row i of sequence s sees cached
+// positions p <= context_lens[s] - n_s + i; fp32 operands and accumulation
+// throughout (v_mfma_f32_16x16x4f32, 256 FLOP per clock and CU, the bound of
+// this kernel).
+//
+// A workgroup (4 waves, two workgroups per CU) takes 64 query rows = bq
+// tokens x G query heads of one kv head, 16 rows per wave, and streams
+// 32-token K/V tiles through a two-stage LDS ring; the global loads of tile
+// k + 1 are in flight while tile k is computed. 64 rows: a prompt of a few
+// hundred tokens still gives each (sequence, head) several items, and the
+// fp32 MFMA is slow enough (32 cycles) that 16 rows per wave already hide the
+// LDS reads. Items are split evenly over the workgroups (prefill_split.h)
+// where the launcher has a workspace.
+//
+// Fragments (lane = 16j + n16): the score MFMAs take K as A (row = token) and
+// Q as B (column = query row), so that the lane ends up with the scores of
+// row n16 at tokens 16h + 4j + e, which are its A operands of P.V as they
+// are. The order of the sum over d and the placement of output columns are
+// free: score MFMA (i, e) takes d = 16i + 4j + e and o[4w + e] holds columns
+// 64w + 4 n16 + e, so every LDS read is 16 bytes and conflict-free.
+//
+// Accuracy: against 64 bits this kernel must not be further off than the
+// VALU form it replaces, whose sums are short per-lane chains joined by
+// trees. A score is therefore a tree over chains of two MFMAs (eight
+// products), and P.V of a tile likewise, added to the running accumulator
+// once per tile (which also folds the rescale into that add). Scores and row
+// maxima stay raw: (s - m) * c rounds an exponent once, by its own size.
+#include "prefill_split.h"
+
+namespace clv {
+namespace {
+
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * 64;
+constexpr int kRows = kWaves * 16;  // query rows per workgroup
+constexpr int kBK = 32;             // K/V tokens per tile
+static_assert(kWaves == 4, "the per-wave flags are read as one word");
+
+// Workgroups (and so waves per SIMD) of a compute unit. More of them at
+// head_dim 64 hide more latency but cut the items into more partials: 8 x 512
+// tokens, 12 heads: 68.7 us at two, 64.2 at three, 85.8 at four; one sequence
+// of 512: 27.1, 32.8 and 46.2 us.
+constexpr int kPerCu = 2;
+
+struct SplitCfg {
+  static constexpr int kBK = clv::kBK;
+  static constexpr int kItemUnits = 1;
+  static constexpr int kMinShare = 3;
+  static constexpr int kCutUnits = 3;
+  static __device__ __forceinline__ int tile_units(int) { return 1; }
+  static __device__ __forceinline__ int snap(int share) { return max(1, share / 16); }
+};
+
+__device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a),
+                                              __builtin_bit_cast(float, b), c, 0, 0, 0);
+}
+
+// Tiles up to which no item is long enough for a cut to pay.
+constexpr int kSplitMinTiles = 6;
+
+template <int D, bool SPLIT>
+__global__ void __launch_bounds__(kThreads, kPerCu)
+chunked_prefill_f32(const PrefillArgs args) {
+  constexpr int NQK = D / 16;            // 16-byte Q / K words per lane
+  constexpr int CH = D / 16;             // output blocks
+  constexpr int ROW = D + 4;             // LDS row stride (floats)
+  constexpr int CPR = D / 4;             // 16-byte chunks per row
+  constexpr int RPP = kThreads / CPR;    // rows per load pass
+  constexpr int PASSES = kBK / RPP;
+  constexpr int WROWS = 64 / CPR;        // rows of one load instruction of a wave
+  __shared__ __attribute__((aligned(16))) float sK[2][kBK * ROW];
+  __shared__ __attribute__((aligned(16))) float sV[2][kBK * ROW];
+  __shared__ __attribute__((aligned(4))) uint8_t sValid[2][kBK];
+  // Per wave: the V rows it staged hold a value that is not finite.
+  __shared__ __attribute__((aligned(4))) uint8_t sInf[2][kWaves];
+  __shared__ int s_pre[SPLIT ? kPrefillSplitItems + 1 : 1];
+  __shared__ int s_tmp[3 * kWaves];
+  __shared__ int s_cur[kWaves][PrefillSched<SplitCfg>::kCursorInts];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15;
+  const int j = lane >> 4;
+  // Consecutive ids go round-robin over the 8 XCDs: give each XCD a
+  // contiguous range of logical work, so that the query tiles of one kv head
+  // share its L2.
+  const int per_xcd = gridDim.x / 8;
+  const int L = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+
+  typedef PrefillSched<SplitCfg> Sched;
+  if constexpr (SPLIT) {
+    Sched sched;
+    sched.init<kThreads>(args.p, args.bq, args.n_qtiles, args.sp.groups, s_pre, s_tmp);
+    sched.start(L, s_cur[wave]);
+    if (tid == 0) reinterpret_cast<PrefillDesc *>(args.sp.desc)[L] = PrefillDesc{-1, 0, 0, 0};
+  } else if (L >= args.total) {
+    return;
+  }
+
+  for (bool first = true;; first = false) {
+    const PrefillArgs ar0 = SPLIT ? reload_args() : args;
+    const PrefillParams &p = ar0.p;
+    const int bq = ar0.bq, n_qtiles = ar0.n_qtiles;
+    PrefillItem it;
+    int t0 = 0, t1, nt;  // this workgroup's tiles of the item, and all of them
+    if constexpr (SPLIT) {
+      if (!Sched::next(p, bq, n_qtiles, s_pre, s_cur[wave], it, t0, t1, nt)) break;
+    } else {
+      if (!first) break;
+      const int qt = n_qtiles - 1 - L % n_qtiles;  // longest query tiles first
+      const int rest = L / n_qtiles;
+      it.set(p, bq, rest / p.num_kv_heads, rest % p.num_kv_heads, qt);
+      if (it.q0 >= it.n_new) break;
+      nt = t1 = Sched::tiles(it.kv_end);
+    }
+    const int G = p.group;
+    // A negative scale flips the sign of Q, a zero one becomes 2^-126 (weights
+    // of 1 to far below fp32 resolution, 0 for masked scores): the softmax
+    // multiplies by c > 0 only.
+    const float c = fmaxf(fabsf(p.scale_log2), 0x1p-126f);
+    const uint32_t qflip = p.scale_log2 < 0.f ? 0x80000000u : 0u;
+
+    const char *kbase = (const char *)p.k_cache + (int64_t)it.kvh * p.kv_stride_head * 4;
+    const char *vbase = (const char *)p.v_cache + (int64_t)it.kvh * p.kv_stride_head * 4;
+    const int kv_end = it.kv_end;
+    const int te = min(t1, (kv_end + kBK - 1) / kBK);  // 0 tokens: no tile at all
+
+    // Q (B operand) of this lane's row 16 wave + n16.
+    u32x4 q[NQK];
+    int lim;  // last visible position of the row (-1: no row)
+    {
+      const int r = 16 * wave + n16;
+      const int tok = it.q0 + r / G;
+      const bool ok = r < bq * G && tok < it.n_new;
+      lim = ok ? it.base_pos + tok : -1;
+      const float *qrow = (const float *)p.q + (int64_t)(it.qs + (ok ? tok : it.q0)) * p.q_stride_token +
+                          (int64_t)(it.kvh * G + (ok ? r % G : 0)) * p.q_stride_head + 4 * j;
+#pragma unroll
+      for (int i = 0; i < NQK; ++i) {
+        q[i] = load_vec<u32x4>(qrow + 16 * i);
+        q[i] ^= qflip;
+        if (!ok) q[i] = (u32x4){0u, 0u, 0u, 0u};
+      }
+    }
+    // Causal limits of the wave's first and last real rows: tiles at or below
+    // the first need no mask, tiles past the last are left out by this wave.
+    const int rows = (it.q_hi - it.q0) * G;
+    int lim_first = -1, te_w = t0;
+    if (16 * wave < rows) {
+      lim_first = it.base_pos + it.q0 + 16 * wave / G;
+      const int lim_last = it.base_pos + it.q0 + min(16 * wave + 15, rows - 1) / G;
+      te_w = max(t0, min(te, lim_last < 0 ? 0 : lim_last / kBK + 1));
+    }
+
+    // Tile loader: thread handles chunk tid % CPR of rows tid / CPR + RPP * i;
+    // the rows of one load instruction lie in one block (block_size >= WROWS).
+    const int lchunk = tid % CPR;
+    const int lrow = tid / CPR;
+    const int wrow = WROWS * wave;
+    const uint32_t sblk32 = (uint32_t)(p.kv_stride_block * 4), stok32 = (uint32_t)(p.kv_stride_token * 4);
+    const uint32_t bmask = (1u << p.block_shift) - 1u;
+    const uint32_t lane_off = (uint32_t)(lrow - wrow) * stok32 + (uint32_t)lchunk * 16u;
+    typedef const int32_t __attribute__((address_space(4))) *cint_t;
+    const cint_t brow = (cint_t)(p.block_tables + (int64_t)it.s * p.max_blocks_per_seq);
+    u32x4 kreg[PASSES], vreg[PASSES];
+    bool rvalid[PASSES];
+    int rblk[PASSES];
+    auto fetch_blocks = [&](int tile) {
+#pragma unroll
+      for (int i = 0; i < PASSES; ++i) {
+        const int t = tile * kBK + wrow + RPP * i;
+        rblk[i] = (tile < te && t < kv_end) ? brow[t >> p.block_shift] : -1;
+      }
+    };
+    // Lanes whose token is not readable (past the context, or in an unmapped
+    // block) read zeros from the buffer resource's range check.
+    auto load_tile = [&](int tile) {
+#pragma unroll
+      for (int i = 0; i < PASSES; ++i) {
+        const uint32_t t = (uint32_t)(tile * kBK + wrow + RPP * i);
+        const bool bok = (unsigned)rblk[i] < (unsigned)p.num_blocks;
+        const bool ok = bok && (int)t + (lrow - wrow) < kv_end;
+        rvalid[i] = ok;
+        const uint64_t boff = (uint64_t)(uint32_t)(bok ? rblk[i] : 0) * sblk32;
+        const int nrec = bok ? (int)(stok32 << p.block_shift) : 0;
+        const uint32_t voff = ok ? (t & bmask) * stok32 + lane_off : 0x80000000u;
+        kreg[i] = buf_load<u32x4>(make_rsrc_range(kbase + boff, nrec), voff);
+        vreg[i] = buf_load<u32x4>(make_rsrc_range(vbase + boff, nrec), voff);
+      }
+    };
+    auto store_tile = [&](int buf) {
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < PASSES; ++i) {
+        const int row = lrow + RPP * i;
+        store_vec<u32x4>(&sK[buf][row * ROW + lchunk * 4], kreg[i]);
+        store_vec<u32x4>(&sV[buf][row * ROW + lchunk * 4], vreg[i]);
+        if (lchunk == 0) sValid[buf][row] = rvalid[i] ? 1 : 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= (vreg[i][e] & 0x7f800000u) == 0x7f800000u;
+      }
+      const bool any_bad = __any(bad);
+      if (lane == 0) sInf[buf][wave] = any_bad ? 1 : 0;
+    };
+
+    f32x4 o[CH];
+    float m_run = kNegInf, l_run = 0.f;
+#pragma unroll
+    for (int m = 0; m < CH; ++m) o[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    fetch_blocks(t0);
+    if (t0 < te) {
+      load_tile(t0);
+      fetch_blocks(t0 + 1);
+      store_tile(t0 & 1);  // the item before this one ended with a barrier
+    }
+    __syncthreads();
+
+    for (int tile = t0; tile < te; ++tile) {
+      const int buf = tile & 1;
+      const bool more = tile + 1 < te;
+      if (more) {
+        load_tile(tile + 1);
+        fetch_blocks(tile + 2);
+      }
+      if (tile < te_w) {
+        // Scores: chains of two MFMAs (eight products), joined by a tree.
+        f32x4 sacc[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          f32x4 part[NQK / 4];  // the tree's level above four words of K
+#pragma unroll
+          for (int i4 = 0; i4 < NQK; i4 += 4) {
+            f32x4 ch[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) ch[u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const u32x4 k =
+                  load_vec<u32x4>(&sK[buf][(16 * h + n16) * ROW + 16 * (i4 + i) + 4 * j]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                ch[4 * (i & 1) + e] = mfma(k[e], q[i4 + i][e], ch[4 * (i & 1) + e]);
+            }
+            part[i4 / 4] = ((ch[0] + ch[1]) + (ch[2] + ch[3])) + ((ch[4] + ch[5]) + (ch[6] + ch[7]));
+          }
+          sacc[h] = NQK == 8 ? part[0] + part[NQK / 4 - 1] : part[0];
+        }
+        const bool full = __all(sValid[buf][lane & 31] != 0) && tile * kBK + kBK - 1 <= lim_first;
+        // Bit 4h + e: the row sees token 16h + 4j + e. Hidden scores become -inf.
+        uint32_t vis = 0xffu;
+        if (!full) {
+          vis = 0;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t vf = *reinterpret_cast<const uint32_t *>(&sValid[buf][16 * h + 4 * j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const uint32_t seen = ((vf >> (8 * e)) & 1u) &
+                                    (tile * kBK + 16 * h + 4 * j + e <= lim ? 1u : 0u);
+              vis |= seen << (4 * h + e);
+              if (seen == 0) sacc[h][e] = kNegInf;
+            }
+          }
+        }
+        float mx = kNegInf;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mx = fmaxf(mx, sacc[h][e]);
+        mx = fmaxf(mx, shfl_xor(mx, 16));
+        mx = fmaxf(mx, shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx);
+        const float msub = m_new == kNegInf ? 0.f : m_new;
+        const float alpha = fast_exp2((m_run - msub) * c);
+        m_run = m_new;
+        float pr[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pr[h][e] = fast_exp2((sacc[h][e] - msub) * c);
+        l_run = l_run * alpha + (((pr[0][0] + pr[0][1]) + (pr[0][2] + pr[0][3])) +
+                                 ((pr[1][0] + pr[1][1]) + (pr[1][2] + pr[1][3])));
+        float ar[4];  // alpha of the accumulator's rows 4j + r
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ar[r] = shfl(alpha, 4 * j + r);
+
+        if (full || *reinterpret_cast<const uint32_t *>(&sInf[buf][0]) == 0) {
+#pragma unroll
+          for (int w = 0; w < CH / 4; ++w) {
+            u32x4 v[2][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int k = 0; k < 4; ++k)
+                v[h][k] = load_vec<u32x4>(&sV[buf][(16 * h + 4 * j + k) * ROW + 64 * w + 4 * n16]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              f32x4 t[2][2];
+#pragma unroll
+              for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) t[h][k] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                  t[h][k & 1] = mfma(__builtin_bit_cast(uint32_t, pr[h][k]), v[h][k][e], t[h][k & 1]);
+              const f32x4 sum = (t[0][0] + t[0][1]) + (t[1][0] + t[1][1]);
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                o[4 * w + e][r] = __builtin_fmaf(o[4 * w + e][r], ar[r], sum[r]);
+            }
+          }
+        } else {
+          // A masked tile with an infinity or NaN in V: a row must not take
+          // 0 * inf from tokens it does not see, so its tokens are added one
+          // by one.
+#pragma unroll
+          for (int m = 0; m < CH; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[m][r] *= ar[r];
+          for (int t = 0; t < kBK; ++t) {
+            float pv = 0.f;
+            uint32_t seen = 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (t == 16 * h + 4 * j + e) {
+                  pv = pr[h][e];
+                  seen = (vis >> (4 * h + e)) & 1u;
+                }
+            const int src = 16 * ((t >> 2) & 3);  // lanes that hold token t
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float a = shfl(pv, src + 4 * j + r);
+              const bool s = __shfl((int)seen, src + 4 * j + r, 64) != 0;
+#pragma unroll
+              for (int m = 0; m < CH; ++m) {
+                const float v = sV[buf][t * ROW + 64 * (m >> 2) + 4 * n16 + (m & 3)];
+                o[m][r] = s ? __builtin_fmaf(a, v, o[m][r]) : o[m][r];
+              }
+            }
+          }
+        }
+      }
+      if (more) store_tile(buf ^ 1);
+      __syncthreads();
+    }
+
+    l_run += shfl_xor(l_run, 16);
+    l_run += shfl_xor(l_run, 32);
+    // The rest of the arguments are read only now.
+    const PrefillArgs ar1 = SPLIT ? reload_args() : args;
+    const bool whole = !SPLIT || (t0 == 0 && t1 == nt);
+    const int64_t prow = (int64_t)(2 * L + (t0 == 0 ? 1 : 0)) * kRows;  // partial's first row
+    if constexpr (SPLIT) {
+      if (!whole) {
+        if (tid == 0) prefill_note(ar1.sp, L, it, t0 == 0, t1 == nt);
+        if (j == 0 && 16 * wave + n16 < rows) {
+          ar1.sp.ws_m[prow + 16 * wave + n16] = m_run;
+          ar1.sp.ws_l[prow + 16 * wave + n16] = l_run;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * wave + 4 * j + r;
+      const float l = shfl(l_run, 4 * j + r);
+      if (row >= rows) continue;
+      const int tok = it.q0 + row / G;
+      float *dst;
+      float inv;
+      if (whole) {
+        // A row at or past max_query_len (a caller error) is marked with NaN.
+        inv = tok >= ar1.p.max_query_len ? __builtin_nanf("") : l > 0.f ? 1.f / l : 0.f;
+        dst = (float *)ar1.p.out + (int64_t)(it.qs + tok) * ar1.p.out_stride_token +
+              (int64_t)(it.kvh * G + row % G) * ar1.p.out_stride_head;
+      } else {
+        inv = 1.f;
+        dst = ar1.sp.ws_o + (prow + row) * D;
+      }
+#pragma unroll
+      for (int w = 0; w < CH / 4; ++w)
+        store_vec<f32x4>(dst + 64 * w + 4 * n16,
+                         (f32x4){o[4 * w][r] * inv, o[4 * w + 1][r] * inv, o[4 * w + 2][r] * inv,
+                                 o[4 * w + 3][r] * inv});
+    }
+    if (t1 == nt && it.qt == ar1.n_qtiles - 1 && it.q_hi < it.n_new)
+      prefill_nan_tail<float, D, kThreads>(ar1.p, it);
+  }
+}
+
+template <int D>
+hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream) {
+  PrefillArgs args{};
+  args.p = p;
+  args.bq = kRows / p.group;
+  args.n_qtiles = max(1, (p.max_query_len + args.bq - 1) / args.bq);
+  const int64_t total = (int64_t)p.num_seqs * p.num_kv_heads * args.n_qtiles;
+  if (total > (int64_t)1 << 30) return hipErrorInvalidValue;
+  if (sp != nullptr) {
+    args.sp = *sp;
+    hipLaunchKernelGGL((chunked_prefill_f32<D, true>), dim3((unsigned)sp->groups), dim3(kThreads),
+                       0, stream, args);
+    hipLaunchKernelGGL((prefill_merge<float, D, kRows>),
+                       dim3((unsigned)sp->groups, kRows / kPrefillMergeRows), dim3(256), 0, stream,
+                       args);
+    return hipGetLastError();
+  }
+  args.total = (int)total;
+  hipLaunchKernelGGL((chunked_prefill_f32<D, false>), dim3((unsigned)((total + 7) / 8 * 8)),
+                     dim3(kThreads), 0, stream, args);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+bool prefill_f32_supported(const PrefillParams &p, int block_size) {
+  // One load instruction of a wave covers 256 / head_dim rows of one block,
+  // and offsets inside a block are 32-bit bytes.
+  const uint64_t lim = (uint64_t)1 << 31;
+  return (p.head_dim == 64 || p.head_dim == 128) && block_size >= 4 && p.group <= kRows &&
+         (uint64_t)p.kv_stride_block * 4 < lim &&
+         ((uint64_t)p.kv_stride_token * 4 << p.block_shift) < lim;
+}
+
+PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p) {
+  return prefill_split_shape(p, kRows, kBK, kPerCu, 1, kSplitMinTiles, false);
+}
+
+hipError_t launch_prefill_f32(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream) {
+  if (p.head_dim == 128) return launch_td<128>(p, sp, stream);
+  if (p.head_dim == 64) return launch_td<64>(p, sp, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace clv

@@ -604,7 +604,11 @@ bool prefill_mfma_supported(DType dt, int head_dim, int block_size) {
          block_size >= 512 / head_dim;
 }
 
-hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, hipStream_t stream) {
+// One workgroup per item only.
+PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &) { return {kRows, 0}; }
+
+hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *,
+                               hipStream_t stream) {
   // The tile loader computes addresses inside a block with 32-bit byte
   // offsets below 2^31; pools with larger blocks take the VALU kernel.
   const uint64_t eb = 2, lim = (uint64_t)1 << 31;

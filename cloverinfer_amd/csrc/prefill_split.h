@@ -1,0 +1,371 @@
+// prefill_split.h - the even split of a chunked prefill over workgroups,
+// shared by the 16-bit and the fp32 MFMA kernels, and the merge of what it
+// cuts.
+//
+// A prefill's work items are (sequence, kv head, query tile); an item runs
+// over the K/V tiles its last row sees. One workgroup per item leaves the
+// chip idle where items are few or uneven: 24 sequences of 0..6000 cached
+// tokens (28/4 heads, 40 % of them bringing 1..300 tokens, the rest one) ran
+// 357 us at 156 TFLOP/s, most of it a few long items alone. Here `groups`
+// workgroups split the items' flattened K/V tiles evenly, as the decode's
+// stream kernel does: group w takes the units [bound(w), bound(w + 1)),
+// crossing item borders, and an item cut by a bound leaves one partial per
+// group in the workspace, which prefill_merge combines.
+//
+// Units: an item costs Cfg::kItemUnits (its Q loads and the fill of the tile
+// ring) plus Cfg::tile_units(rows) per K/V tile. The items of one kv head
+// follow each other, a sequence's query tiles in folded order (heaviest,
+// lightest, second heaviest, ...), so that equal shares of a uniform batch
+// tend to end at item borders; a bound within Cfg::snap() units of an item
+// border moves onto it, as a cut costs two partials and their merge. snap() is
+// at least kItemUnits and the units of a tile, so that every group between
+// an item's first and last one holds at least one of its tiles. Where every
+// group gets at most one item and the longest is not far above the even
+// share, nothing is cut at all: the cuts (kCutUnits: what a cut group loses to
+// its two partials and their merge) would cost more than the evenness gives.
+#pragma once
+
+#include "attn_common.h"
+
+namespace clv {
+
+// What a group left in the workspace: the item whose first part it holds
+// (s < 0: none; partial slot 2w + 1), and whether its first item was begun
+// by an earlier group (cont, partial slot 2w) and ends here.
+struct __attribute__((aligned(16))) PrefillDesc {
+  int32_t s, kvh, qt;
+  int32_t cont;  // 0: none, 1: goes on in the next group, 2: ends here
+};
+
+// One work item.
+struct PrefillItem {
+  int s, kvh, qt;
+  int qs, n_new;         // first query row of the sequence, its rows
+  int q0, q_hi;          // rows [q0, q_hi) of the chunk
+  int ctx, base_pos;     // cached tokens; position of row 0
+  int kv_end;            // tokens the last row sees
+
+  __device__ __forceinline__ void set(const PrefillParams &p, int bq, int s_, int kvh_, int qt_) {
+    s = s_;
+    kvh = kvh_;
+    qt = qt_;
+    qs = p.query_start_loc[s];
+    n_new = p.query_start_loc[s + 1] - qs;
+    const int cap = p.max_blocks_per_seq << p.block_shift;
+    ctx = max(0, min(p.context_lens[s], cap));
+    base_pos = ctx - n_new;
+    q0 = qt * bq;
+    q_hi = min(q0 + bq, n_new);
+    kv_end = max(0, min(ctx, base_pos + q_hi));
+  }
+};
+
+template <class Cfg>
+struct PrefillSched {
+  static constexpr int kCursorInts = 5;
+  const int *pre;  // LDS: exclusive prefix of the units of one kv head's items
+  int n;           // entries: num_seqs * nq
+  int nq;          // query tiles per sequence the entries allow for
+  int C, N, W;     // units per kv head, units in all, groups in use
+  int tol;
+  bool whole;      // nothing is cut: one item per group, one unit per item
+
+  // Query tile at position pos of a sequence's nqs tiles.
+  static __device__ __forceinline__ int folded(int pos, int nqs) {
+    return (pos & 1) ? pos >> 1 : nqs - 1 - (pos >> 1);
+  }
+  static __device__ __forceinline__ int tiles(int kv_end) {
+    return max(1, (kv_end + Cfg::kBK - 1) / Cfg::kBK);
+  }
+  static __device__ __forceinline__ int seq_tiles(int n_new, int bq, int nq) {
+    return min(nq, (max(0, n_new) + bq - 1) / bq);
+  }
+
+  // Fills buf (kPrefillSplitItems + 1 ints of LDS; tmp: 3 per wave) and the
+  // totals; every thread of the workgroup (NT of them) calls it.
+  template <int NT>
+  __device__ __forceinline__ void init(const PrefillParams &p, int bq, int nq_, int groups,
+                                       int *buf, int *tmp) {
+    nq = nq_;
+    n = p.num_seqs * nq;
+    pre = buf;
+    const int tid = threadIdx.x;
+    const int per = (n + NT - 1) / NT;
+    const int b = min(n, tid * per), e = min(n, b + per);
+    int units = 0, count = 0, most = 0;
+    for (int i = b; i < e; ++i) {
+      const int s = i / nq, pos = i - s * nq;
+      PrefillItem it;
+      it.set(p, bq, s, 0, 0);
+      const int nqs = seq_tiles(it.n_new, bq, nq);
+      int u = 0;
+      if (pos < nqs) {
+        it.set(p, bq, s, 0, folded(pos, nqs));
+        u = Cfg::kItemUnits + tiles(it.kv_end) * Cfg::tile_units((it.q_hi - it.q0) * p.group);
+        ++count;
+      }
+      buf[i] = u;
+      units += u;
+      most = max(most, u);
+    }
+    // Inclusive scans over the wave, then over the waves' totals.
+    int xu = units, xc = count;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int yu = __shfl_up(xu, off, 64), yc = __shfl_up(xc, off, 64);
+      if ((tid & 63) >= off) {
+        xu += yu;
+        xc += yc;
+      }
+      most = max(most, __shfl_xor(most, off, 64));
+    }
+    if ((tid & 63) == 63) {
+      tmp[3 * (tid >> 6)] = xu;
+      tmp[3 * (tid >> 6) + 1] = xc;
+      tmp[3 * (tid >> 6) + 2] = most;
+    }
+    __syncthreads();
+    int ru = xu - units, rc = xc - count;
+    int tu = 0, tc = 0;
+    most = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+      if (w < (tid >> 6)) {
+        ru += tmp[3 * w];
+        rc += tmp[3 * w + 1];
+      }
+      tu += tmp[3 * w];
+      tc += tmp[3 * w + 1];
+      most = max(most, tmp[3 * w + 2]);
+    }
+    const int H = p.num_kv_heads;
+    const int share = tu * H / min(groups, max(1, tu * H / Cfg::kMinShare));
+    whole = tc * H <= groups && most <= share + share / 4 + Cfg::kCutUnits;
+    int run = whole ? rc : ru;
+    for (int i = b; i < e; ++i) {
+      const int u = buf[i];
+      buf[i] = run;
+      run += whole ? (u > 0 ? 1 : 0) : u;
+    }
+    if (tid == 0) buf[n] = whole ? tc : tu;
+    __syncthreads();
+    C = __builtin_amdgcn_readfirstlane(whole ? tc : tu);
+    N = C * H;
+    W = whole ? N : min(groups, max(1, N / Cfg::kMinShare));
+    tol = whole ? 0 : Cfg::snap(share);
+  }
+
+  // Entry holding unit rem of a kv head (0 <= rem < C): the last one with
+  // pre[i] <= rem; 64 candidates a round, as in the decode's stream kernel.
+  __device__ __forceinline__ int find(int rem) const {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, len = n;
+    while (len > 1) {
+      const int stride = (len + 63) / 64;
+      const bool le = lane * stride < len && pre[lo + lane * stride] <= rem;
+      const int k = 63 - __builtin_clzll(__ballot(le));
+      lo += k * stride;
+      len = min(stride, len - k * stride);
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+  }
+
+  // First unit of group w. Never decreases in w: a bound only moves onto the
+  // item border nearest to it.
+  __device__ __forceinline__ int bound(int w) const {
+    if (w <= 0) return 0;
+    if (w >= W) return N;
+    const int x = (int)((int64_t)w * N / W);
+    const int kvh = x / C, rem = x - kvh * C;
+    const int i = find(rem);
+    const int lo = __builtin_amdgcn_readfirstlane(pre[i]);
+    const int hi = __builtin_amdgcn_readfirstlane(pre[i + 1]);
+    const int dl = rem - lo, dh = hi - rem;
+    if (min(dl, dh) > tol) return x;
+    return kvh * C + (dl <= dh ? lo : hi);
+  }
+
+  // Writes the cursor of group w, kCursorInts ints of LDS that only this
+  // wave uses.
+  __device__ __forceinline__ void start(int w, int *cur) const {
+    int x = 0, x_end = 0, entry = 0;
+    if (N > 0 && w < W) {
+      x = bound(w);
+      x_end = bound(w + 1);
+      if (x < x_end) entry = find(x % C);
+    }
+    if ((threadIdx.x & 63) == 0) {
+      cur[0] = x;
+      cur[1] = x_end;
+      cur[2] = entry;
+      cur[3] = C;
+      cur[4] = whole ? 1 : 0;
+    }
+  }
+
+  // Next piece of the group: tiles [t0, t1) of the nt tiles of item it (an
+  // item of no tokens counts one); false when the group is done. The cursor
+  // lives in LDS because the kernels' tile loops leave it no registers.
+  static __device__ __forceinline__ bool next(const PrefillParams &p, int bq, int nq,
+                                              const int *pre, int *cur, PrefillItem &it, int &t0,
+                                              int &t1, int &nt) {
+    int x = __builtin_amdgcn_readfirstlane(cur[0]);
+    const int x_end = __builtin_amdgcn_readfirstlane(cur[1]);
+    int entry = __builtin_amdgcn_readfirstlane(cur[2]);
+    const int C = __builtin_amdgcn_readfirstlane(cur[3]);
+    const bool whole = __builtin_amdgcn_readfirstlane(cur[4]) != 0;
+    bool found = false;
+    while (!found && x < x_end) {
+      const int kvh = x / C;
+      const int rem = x - kvh * C;
+      if (rem == 0) entry = 0;  // a kv head's first item
+      while (__builtin_amdgcn_readfirstlane(pre[entry + 1]) <= rem) ++entry;
+      const int s = entry / nq;
+      const int lo = kvh * C + __builtin_amdgcn_readfirstlane(pre[entry]);
+      const int hi = kvh * C + __builtin_amdgcn_readfirstlane(pre[entry + 1]);
+      const int n_new = p.query_start_loc[s + 1] - p.query_start_loc[s];
+      it.set(p, bq, s, kvh, folded(entry - s * nq, seq_tiles(n_new, bq, nq)));
+      nt = tiles(it.kv_end);
+      const int u = Cfg::tile_units((it.q_hi - it.q0) * p.group);
+      const int end = min(x_end, hi);
+      const int first = lo + Cfg::kItemUnits;
+      t0 = whole ? 0 : min((max(0, x - first) + u - 1) / u, nt);
+      t1 = whole ? nt : min((max(0, end - first) + u - 1) / u, nt);
+      x = end;
+      ++entry;
+      found = t0 < t1;
+    }
+    if ((threadIdx.x & 63) == 0) {
+      cur[0] = x;
+      cur[2] = entry;
+    }
+    return found;
+  }
+};
+
+// The kernel's argument, read again from where the launch left it: values
+// that a long loop does not use are then not kept (or spilled) across it.
+// `args` must be the kernel's first and only argument.
+__device__ __forceinline__ PrefillArgs reload_args() {
+  typedef const PrefillArgs __attribute__((address_space(4))) *args_t;
+  args_t a = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  PrefillArgs r;
+  __builtin_memcpy(&r, (const PrefillArgs *)a, sizeof(r));
+  return r;
+}
+
+// Records the partial that group w leaves of item `it`: its first part, or a
+// later one that ends the item or not. One thread writes all of a group's.
+__device__ __forceinline__ void prefill_note(const PrefillSplit &sp, int w, const PrefillItem &it,
+                                             bool begins, bool ends) {
+  PrefillDesc *d = reinterpret_cast<PrefillDesc *>(sp.desc) + w;
+  if (begins) {
+    d->s = it.s;
+    d->kvh = it.kvh;
+    d->qt = it.qt;
+  } else {
+    d->cont = ends ? 2 : 1;
+  }
+}
+
+// Merges the partials of the items that the split cut: workgroup (w, y)
+// takes rows [y * kMergeRows, ..) of the item that group w begins and does
+// not finish. Bound by the partials' bytes; LPR lanes share a row (16 bytes
+// each), lane k of them weighs partial k, so that weights cost one round trip
+// for up to LPR partials.
+constexpr int kPrefillMergeRows = 32;
+
+template <typename T, int D, int ROWS>
+__global__ void __launch_bounds__(256)
+prefill_merge(const PrefillArgs args) {
+  const PrefillParams &p = args.p;
+  const PrefillSplit &sp = args.sp;
+  const int bq = args.bq;
+  constexpr int LPR = D / 4;
+  constexpr int RPP = 256 / LPR;
+  static_assert(ROWS % kPrefillMergeRows == 0 || ROWS < kPrefillMergeRows, "row chunks");
+  const PrefillDesc *desc = (const PrefillDesc *)sp.desc;
+  const int w = blockIdx.x;
+  const PrefillDesc d = desc[w];
+  if (d.s < 0) return;
+  const int lane = threadIdx.x & 63;
+  int n = 1;
+  for (int b = w + 1; b < sp.groups; b += 64) {
+    const uint64_t ends = __ballot(b + lane < sp.groups && desc[b + lane].cont == 2);
+    if (ends != 0) {
+      n = b - w + __builtin_ctzll(ends) + 1;
+      break;
+    }
+  }
+  PrefillItem it;
+  it.set(p, bq, d.s, d.kvh, d.qt);
+  const int G = p.group;
+  const int rows = (it.q_hi - it.q0) * G;
+  const int sub = threadIdx.x % LPR;
+  const int r_end = min(rows, (int)(blockIdx.y + 1) * kPrefillMergeRows);
+  for (int r = blockIdx.y * kPrefillMergeRows + threadIdx.x / LPR; r < r_end; r += RPP) {
+    auto row_of = [&](int k) {  // row of partial k in the workspace
+      return (int64_t)(k == 0 ? 2 * w + 1 : 2 * (w + k)) * ROWS + r;
+    };
+    const float c = fmaxf(fabsf(p.scale_log2), 0x1p-126f);  // as the kernels scale scores
+    float M = kNegInf;
+    for (int k = sub; k < n; k += LPR) M = fmaxf(M, sp.ws_m[row_of(k)]);
+#pragma unroll
+    for (int off = 1; off < LPR; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, LPR));
+    const float Msub = M == kNegInf ? 0.f : M;
+    float L = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < n; k0 += LPR) {
+      const int cnt = min(LPR, n - k0);
+      float wk = 0.f;
+      if (sub < cnt) {
+        wk = fast_exp2((sp.ws_m[row_of(k0 + sub)] - Msub) * c);
+        L += sp.ws_l[row_of(k0 + sub)] * wk;
+      }
+      for (int k = 0; k < cnt; k += 4) {  // four rows' loads in flight
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          v[u] = load_vec<f32x4>(sp.ws_o + row_of(k0 + min(k + u, cnt - 1)) * D + 4 * sub);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float f = __shfl(wk, min(k + u, LPR - 1), LPR);
+          if (k + u < cnt) acc += v[u] * f;
+        }
+      }
+    }
+#pragma unroll
+    for (int off = 1; off < LPR; off <<= 1) L += __shfl_xor(L, off, LPR);
+    const int tok = it.q0 + r / G;
+    const float inv = tok >= p.max_query_len ? __builtin_nanf("") : L > 0.f ? 1.f / L : 0.f;
+    T *dst = (T *)p.out + (int64_t)(it.qs + tok) * p.out_stride_token +
+             (int64_t)(d.kvh * G + r % G) * p.out_stride_head + 4 * sub;
+    if constexpr (sizeof(T) == 4) {
+      store_vec<f32x4>(dst, acc * inv);
+    } else {
+      uint32_t h[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) h[e] = __builtin_bit_cast(uint16_t, (T)(acc[e] * inv));
+      store_vec<u32x2>(dst, (u32x2){h[0] | (h[1] << 16), h[2] | (h[3] << 16)});
+    }
+  }
+}
+
+// Rows past the grid's query tiles (a chunk longer than max_query_len, a
+// caller error) are filled with NaN by the workgroup of the last tile, so
+// that the error shows in the output instead of stale memory.
+template <typename T, int D, int NT>
+__device__ __forceinline__ void prefill_nan_tail(const PrefillParams &p, const PrefillItem &it) {
+  const T nan = (T)__builtin_nanf("");
+  const int G = p.group;
+  for (int idx = threadIdx.x; idx < (it.n_new - it.q_hi) * G * D; idx += NT) {
+    const int d = idx % D;
+    const int h = (idx / D) % G;
+    const int tok = it.q_hi + idx / (D * G);
+    ((T *)p.out)[(int64_t)(it.qs + tok) * p.out_stride_token +
+                 (int64_t)(it.kvh * G + h) * p.out_stride_head + d] = nan;
+  }
+}
+
+}  // namespace clv

@@ -685,4 +685,13 @@ def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     a.num_blocks = num_blocks
     a.dtype = _dtype_code(q)
     a.scale = float(scale)
-    _native.check(_native.load().clv_chunked_prefill(a, _stream(dev)), "clv_chunked_prefill")
+    lib = _native.load()
+    nbytes = lib.clv_prefill_workspace_bytes(a)
+    if nbytes:
+        # From the caching allocator, on the launch's stream: its memory may be
+        # handed out again once this call's kernels are queued ahead.
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        _native.check(lib.clv_chunked_prefill_split(a, ws.data_ptr(), nbytes, _stream(dev)),
+                      "clv_chunked_prefill_split")
+        return
+    _native.check(lib.clv_chunked_prefill(a, _stream(dev)), "clv_chunked_prefill")

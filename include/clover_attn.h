@@ -347,6 +347,24 @@ int32_t clv_default_num_waves_fp8(void);
  */
 int clv_chunked_prefill(const clv_prefill_args *args, clv_stream_t stream);
 
+/*
+ * The same attention with the work of every sequence, kv head and query tile
+ * split evenly over the compute units: items that the split cuts leave fp32
+ * partials in the workspace, and a second kernel merges them. Equal to
+ * clv_chunked_prefill up to the rounding of that merge. `workspace`: at least
+ * clv_prefill_workspace_bytes(args) bytes, 256-byte aligned, need not be
+ * initialised, free again once the call's work on `stream` is done
+ * (CLV_EWORKSPACE if missing or too small); where that size is 0 the call is
+ * clv_chunked_prefill and the workspace may be null. No counterpart in the
+ * reference.
+ */
+int clv_chunked_prefill_split(const clv_prefill_args *args, void *workspace,
+                              size_t workspace_bytes, clv_stream_t stream);
+
+/* Workspace bytes of clv_chunked_prefill_split: a function of the argument
+ * block's sizes; 0 where the call is not split or the arguments are refused. */
+size_t clv_prefill_workspace_bytes(const clv_prefill_args *args);
+
 #ifdef __cplusplus
 } /* extern "C" */
 #endif
