@@ -44,7 +44,14 @@
 // of tile k - 1 still reads its V; block-table entries are fetched one tile
 // earlier still. Workgroup ids are remapped so that all query tiles of one
 // (sequence, kv head) run on the same XCD and share its L2.
-#include "attn_common.h"
+//
+// Uneven batches run in the split form (prefill_split.h): a workgroup per
+// compute unit takes an even share of the items' tiles, cutting long items.
+// 24 sequences of 0..6000 cached tokens, 60 % of them bringing one token and
+// the rest up to 300 (28/4 heads, bf16): 357 -> 136 us. A wave without rows
+// only stages tiles in either form (one prompt of 777 tokens, 32 heads, whose
+// last query tile has 9 of 256 rows: 36.4 -> 32.1 us).
+#include "prefill_split.h"
 
 #include <type_traits>
 
@@ -108,9 +115,22 @@ __host__ __device__ inline int dispatch_slot(int i, int per_xcd, int valid, int 
   return r0 + (u % heads) * n_q + u / heads;
 }
 
-template <typename T, int D>
+// Units of the split (prefill_split.h): a quarter of the time of a full tile.
+struct SplitCfg {
+  static constexpr int kBK = clv::kBK;
+  static constexpr int kItemUnits = 4;
+  static constexpr int kMinShare = 16;
+  static constexpr int kCutUnits = 40;
+  static __device__ __forceinline__ int tile_units(int rows) { return rows > 128 ? 4 : 2; }
+  static __device__ __forceinline__ int snap(int share) { return max(4, share / 16); }
+};
+
+// Tiles up to which no item is long enough for a cut to pay.
+constexpr int kSplitMinTiles = 16;
+
+template <typename T, int D, bool SPLIT>
 __global__ void __launch_bounds__(kThreads)
-chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
+chunked_prefill_mfma(const PrefillArgs args) {
   typedef Mfma16x16x32<T> MfQK;
   typedef Mfma16x16x32<_Float16> MfPV;
   typedef typename MfQK::op_t qk_t;
@@ -133,30 +153,49 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
   __shared__ __attribute__((aligned(16))) uint16_t sV[3][kBK * VROW];
   __shared__ __attribute__((aligned(4))) uint8_t sValid[3][kBK];  // 1 = the token's block is readable
   __shared__ int sOvf;  // set when a bf16 V value did not fit fp16
+  __shared__ int s_pre[SPLIT ? kPrefillSplitItems + 1 : 1];
+  __shared__ int s_tmp[3 * kWaves];
+  __shared__ int s_cur[kWaves][PrefillSched<SplitCfg>::kCursorInts];
 
   // XCD-aware remap: consecutive ids go round-robin over the 8 XCDs; give
   // each XCD a contiguous range of logical work items, in the order
   // dispatch_slot sets.
   const int per_xcd = gridDim.x / 8;
   const int xcd0 = (blockIdx.x % 8) * per_xcd;
-  const int L = xcd0 + dispatch_slot(blockIdx.x / 8, per_xcd, total - xcd0, n_qtiles,
-                                     p.cus_per_xcd);
-  if (L >= total) return;
-  const int qt = n_qtiles - 1 - L % n_qtiles;  // longest query tiles first
-  const int rest = L / n_qtiles;
-  const int kvh = rest % p.num_kv_heads;
-  const int s = rest / p.num_kv_heads;
+  const int L = SPLIT ? xcd0 + blockIdx.x / 8
+                      : xcd0 + dispatch_slot(blockIdx.x / 8, per_xcd, args.total - xcd0,
+                                             args.n_qtiles, args.p.cus_per_xcd);
+  typedef PrefillSched<SplitCfg> Sched;
+  int *cur = s_cur[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+  if constexpr (SPLIT) {
+    Sched sched;
+    sched.init<kThreads>(args.p, args.bq, args.n_qtiles, args.sp.groups, s_pre, s_tmp);
+    sched.start(L, cur);
+    if (threadIdx.x == 0)
+      reinterpret_cast<PrefillDesc *>(args.sp.desc)[L] = PrefillDesc{-1, 0, 0, 0};
+  } else if (L >= args.total) {
+    return;
+  }
 
-  const int qs = p.query_start_loc[s];
-  const int n_new = p.query_start_loc[s + 1] - qs;
-  const int q0 = qt * bq;
-  if (q0 >= n_new) return;
-  const int cap = p.max_blocks_per_seq << p.block_shift;
-  const int ctx = max(0, min(p.context_lens[s], cap));
-  const int base_pos = ctx - n_new;  // cached position of query 0
-  const int q_hi = min(q0 + bq, n_new);
-  const int kv_end = max(0, min(ctx, base_pos + q_hi));
-  const int ntiles = (kv_end + kBK - 1) / kBK;
+  for (bool first = true;; first = false) {
+  const PrefillArgs ar0 = SPLIT ? reload_args() : args;
+  const PrefillParams &p = ar0.p;
+  const int bq = ar0.bq, n_qtiles = ar0.n_qtiles;
+  PrefillItem it;
+  int t0 = 0, t1, nt;  // this workgroup's tiles of the item, and all of them
+  if constexpr (SPLIT) {
+    if (!Sched::next(p, bq, n_qtiles, s_pre, cur, it, t0, t1, nt)) break;
+  } else {
+    if (!first) break;
+    const int qt = n_qtiles - 1 - L % n_qtiles;  // longest query tiles first
+    const int rest = L / n_qtiles;
+    it.set(p, bq, rest / p.num_kv_heads, rest % p.num_kv_heads, qt);
+    if (it.q0 >= it.n_new) break;
+    nt = t1 = Sched::tiles(it.kv_end);
+  }
+  const int s = it.s, kvh = it.kvh, qs = it.qs, n_new = it.n_new, q0 = it.q0;
+  const int base_pos = it.base_pos, kv_end = it.kv_end;
+  const int te = min(t1, (kv_end + kBK - 1) / kBK);  // tiles [t0, te); no tokens: none
   const int G = p.group;
 
   const int tid = threadIdx.x;
@@ -205,6 +244,8 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
   const int wave_row0 = kWaveRows * wave;
   const int wave_lim = (wave_row0 < bq * G && q0 + wave_row0 / G < n_new)
                            ? base_pos + q0 + wave_row0 / G : -1;
+  // A wave without rows only helps to stage the tiles.
+  const bool active = wave_row0 < (it.q_hi - q0) * G;
 
   // Tile loader: thread handles chunk (tid % CPR) of rows tid / CPR + RPP*i.
   // One load instruction of a wave covers WROWS consecutive rows, which lie
@@ -230,8 +271,8 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
   auto fetch_blocks = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-      const int t0 = tile * kBK + wrow + RPP * i;
-      rblk[i] = (tile < ntiles && t0 < kv_end) ? brow[t0 >> kv.block_shift] : -1;
+      const int tok0 = tile * kBK + wrow + RPP * i;
+      rblk[i] = (tile < te && tok0 < kv_end) ? brow[tok0 >> kv.block_shift] : -1;
     }
   };
   // Rows are read through a buffer resource whose range is the rows of one
@@ -241,13 +282,13 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
   auto load_tile = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-      const uint32_t t0 = (uint32_t)(tile * kBK + wrow + RPP * i);
+      const uint32_t tok0 = (uint32_t)(tile * kBK + wrow + RPP * i);
       const bool bok = (unsigned)rblk[i] < kv.num_blocks;
-      const bool ok = bok && (int)t0 + (lrow - wrow) < kv_end;
+      const bool ok = bok && (int)tok0 + (lrow - wrow) < kv_end;
       rvalid[i] = ok;
       const uint64_t boff = (uint64_t)(uint32_t)(bok ? rblk[i] : 0) * sblk32;
       const int nrec = bok ? (int)(stok32 << kv.block_shift) : 0;
-      const uint32_t voff = ok ? (t0 & bmask) * stok32 + lane_off : 0x80000000u;
+      const uint32_t voff = ok ? (tok0 & bmask) * stok32 + lane_off : 0x80000000u;
       kreg[i] = buf_load<u32x4>(make_rsrc_range(kv.kbase + boff, nrec), voff);
       vreg[i] = buf_load<u32x4>(make_rsrc_range(kv.vbase + boff, nrec), voff);
     }
@@ -476,49 +517,62 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
     // race a slower wave's read, and waves that disagreed on running the
     // exact pass would wait at different barriers.
     if (!EXACT && tid == 0) sOvf = 0;
-    fetch_blocks(0);
-    if (ntiles > 0) {
-      load_tile(0);
-      fetch_blocks(1);
+    fetch_blocks(t0);
+    if (t0 < te) {
+      load_tile(t0);
+      fetch_blocks(t0 + 1);
       __syncthreads();  // sOvf cleared (and the previous pass done with LDS)
-      store_tile(0, exact_c);
+      store_tile(t0 % 3, exact_c);
     }
     __syncthreads();
 
     const bool lag = wave >= kWaves / 2;  // softmax one step behind
     bool full_prev = false;
-    for (int tile = 0; tile < ntiles; ++tile) {
-      const bool more = tile + 1 < ntiles;
-      if (more) load_tile(tile + 1);  // block ids fetched last iteration
-      const bool full = tile_full(tile);
-      const int g = 2 * tile;
-      // The MFMA phases run at raised wave priority: the SIMD's arbiter then
-      // issues the next MFMA as soon as the matrix core takes it, and the
-      // other wave's softmax fills the issue slots in between.
-      if (lag && tile > 0) softmax_step(g - 1, full_prev);
-      __builtin_amdgcn_s_setprio(1);
-      qk(g);
-      if (tile > 0) pv(g - 1);
-      __builtin_amdgcn_s_setprio(0);
-      // Block-table entries for the tile after next, issued before a softmax
-      // (VALU only on full tiles): the scalar loads share the LDS wait
-      // counter, so issued right before an LDS read they would be waited for
-      // there.
-      if (more) fetch_blocks(tile + 2);
-      softmax_step(g, full);
-      __builtin_amdgcn_s_setprio(1);
-      qk(g + 1);
-      pv(g);
-      __builtin_amdgcn_s_setprio(0);
-      if (!lag) softmax_step(g + 1, full);
-      full_prev = full;
+    if (!active) {
+      // A loop of its own: as a branch inside the loop below it cost 120
+      // spilled VGPRs.
+      for (int tile = t0; tile < te; ++tile) {
+        if (tile + 1 < te) {
+          load_tile(tile + 1);
+          fetch_blocks(tile + 2);
+          store_tile((tile + 1) % 3, exact_c);
+        }
+        __syncthreads();
+      }
+    } else {
+      for (int tile = t0; tile < te; ++tile) {
+        const bool more = tile + 1 < te;
+        if (more) load_tile(tile + 1);  // block ids fetched last iteration
+        const bool full = tile_full(tile);
+        const int g = 2 * tile;
+        // The MFMA phases run at raised wave priority: the SIMD's arbiter then
+        // issues the next MFMA as soon as the matrix core takes it, and the
+        // other wave's softmax fills the issue slots in between.
+        if (lag && tile > t0) softmax_step(g - 1, full_prev);
+        __builtin_amdgcn_s_setprio(1);
+        qk(g);
+        if (tile > t0) pv(g - 1);
+        __builtin_amdgcn_s_setprio(0);
+        // Block-table entries for the tile after next, issued before a softmax
+        // (VALU only on full tiles): the scalar loads share the LDS wait
+        // counter, so issued right before an LDS read they would be waited for
+        // there.
+        if (more) fetch_blocks(tile + 2);
+        softmax_step(g, full);
+        __builtin_amdgcn_s_setprio(1);
+        qk(g + 1);
+        pv(g);
+        __builtin_amdgcn_s_setprio(0);
+        if (!lag) softmax_step(g + 1, full);
+        full_prev = full;
 
-      if (more) store_tile((tile + 1) % 3, exact_c);
-      __syncthreads();
-    }
-    if (ntiles > 0) {
-      if (lag) softmax_step(2 * ntiles - 1, full_prev);
-      pv(2 * ntiles - 1);
+        if (more) store_tile((tile + 1) % 3, exact_c);
+        __syncthreads();
+      }
+      if (t0 < te) {
+        if (lag) softmax_step(2 * te - 1, full_prev);
+        pv(2 * te - 1);
+      }
     }
     if constexpr (kBf16 && !EXACT) {
       // A bf16 V value that did not fit fp16 became an infinity (or was
@@ -543,57 +597,75 @@ chunked_prefill_mfma(const PrefillParams p, int bq, int n_qtiles, int total) {
     if (overflow) run_tiles(std::true_type{});
   }
 
-  // ---- normalise and store rows kWaveRows*w + 16rt + 4j + e
+  // ---- normalise and store rows kWaveRows*w + 16rt + 4j + e, or leave them
+  // as a partial (unnormalised) where the split cut the item
+  const PrefillArgs ar1 = SPLIT ? reload_args() : args;
+  const bool whole = !SPLIT || (t0 == 0 && t1 == nt);
+  const int64_t prow = (int64_t)(2 * L + (t0 == 0 ? 1 : 0)) * kRows;
+  if (SPLIT && !whole && tid == 0) prefill_note(ar1.sp, L, it, t0 == 0, t1 == nt);
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
+    if (SPLIT && !whole && j == 0)
+      ar1.sp.ws_m[prow + kWaveRows * wave + 16 * rt + n16] = m_run[rt];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float l = lsum[rt][e];
       const int row = kWaveRows * wave + 16 * rt + 4 * j + e;
       const int tok = q0 + row / G;
-      if (row >= bq * G || tok >= n_new) continue;
-      // A row at or past max_query_len (a caller error) is marked with NaN.
-      const float inv = tok >= p.max_query_len ? __builtin_nanf("") : l > 0.f ? 1.f / l : 0.f;
+      if (row >= ar1.bq * G || tok >= n_new) continue;
       // Lane n16 of MFMA m holds column d = 16m + n16.
-      T *dst = (T *)p.out + (int64_t)(qs + tok) * p.out_stride_token +
-               (int64_t)(kvh * G + row % G) * p.out_stride_head + n16;
+      if (whole) {
+        // A row at or past max_query_len (a caller error) is marked with NaN.
+        const float inv =
+            tok >= ar1.p.max_query_len ? __builtin_nanf("") : l > 0.f ? 1.f / l : 0.f;
+        T *dst = (T *)ar1.p.out + (int64_t)(qs + tok) * ar1.p.out_stride_token +
+                 (int64_t)(kvh * G + row % G) * ar1.p.out_stride_head + n16;
 #pragma unroll
-      for (int m = 0; m < CH; ++m) dst[16 * m] = (T)(o[rt][m][e] * inv);
+        for (int m = 0; m < CH; ++m) dst[16 * m] = (T)(o[rt][m][e] * inv);
+      } else {
+        if (n16 == 0) ar1.sp.ws_l[prow + row] = l;
+        float *dst = ar1.sp.ws_o + (prow + row) * D + n16;
+#pragma unroll
+        for (int m = 0; m < CH; ++m) dst[16 * m] = o[rt][m][e];
+      }
     }
   }
-
-  // Rows past the grid's query tiles (a chunk longer than max_query_len, a
-  // caller error) are filled with NaN by the workgroup of the last tile, so
-  // that the error shows in the output instead of stale memory.
-  if (qt == n_qtiles - 1 && q_hi < n_new) {
-    const T nan = (T)__builtin_nanf("");
-    for (int idx = tid; idx < (n_new - q_hi) * G * D; idx += kThreads) {
-      const int d = idx % D;
-      const int h = (idx / D) % G;
-      const int tok = q_hi + idx / (D * G);
-      ((T *)p.out)[(int64_t)(qs + tok) * p.out_stride_token +
-                   (int64_t)(kvh * G + h) * p.out_stride_head + d] = nan;
-    }
+  if (t1 == nt && it.qt == ar1.n_qtiles - 1 && it.q_hi < n_new)
+    prefill_nan_tail<T, D, kThreads>(ar1.p, it);
+  // Every wave has read sOvf before the next item clears it.
+  if constexpr (SPLIT && kBf16) __syncthreads();
   }
 }
 
-template <typename T>
-hipError_t launch_t(const PrefillParams &p, hipStream_t stream) {
-  const int bq = kRows / p.group;
+template <typename T, int D>
+hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream) {
+  PrefillArgs args{};
+  args.p = p;
+  args.bq = kRows / p.group;
   // At least one query tile per (sequence, kv head): its workgroup marks the
   // rows of chunks longer than max_query_len (see the kernel's end).
-  const int n_qtiles = max(1, (p.max_query_len + bq - 1) / bq);
-  const int64_t total = (int64_t)p.num_seqs * p.num_kv_heads * n_qtiles;
+  args.n_qtiles = max(1, (p.max_query_len + args.bq - 1) / args.bq);
+  const int64_t total = (int64_t)p.num_seqs * p.num_kv_heads * args.n_qtiles;
   if (total <= 0) return hipSuccess;
   if (total > (int64_t)1 << 30) return hipErrorInvalidValue;
-  const unsigned grid = (unsigned)((total + 7) / 8 * 8);
-  if (p.head_dim == 128)
-    hipLaunchKernelGGL((chunked_prefill_mfma<T, 128>), dim3(grid), dim3(kThreads), 0, stream, p,
-                       bq, n_qtiles, (int)total);
-  else
-    hipLaunchKernelGGL((chunked_prefill_mfma<T, 64>), dim3(grid), dim3(kThreads), 0, stream, p,
-                       bq, n_qtiles, (int)total);
+  if (sp != nullptr) {
+    args.sp = *sp;
+    hipLaunchKernelGGL((chunked_prefill_mfma<T, D, true>), dim3((unsigned)sp->groups),
+                       dim3(kThreads), 0, stream, args);
+    hipLaunchKernelGGL((prefill_merge<T, D, kRows>),
+                       dim3((unsigned)sp->groups, kRows / kPrefillMergeRows), dim3(256), 0, stream,
+                       args);
+    return hipGetLastError();
+  }
+  args.total = (int)total;
+  hipLaunchKernelGGL((chunked_prefill_mfma<T, D, false>), dim3((unsigned)((total + 7) / 8 * 8)),
+                     dim3(kThreads), 0, stream, args);
   return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_t(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream) {
+  return p.head_dim == 128 ? launch_td<T, 128>(p, sp, stream) : launch_td<T, 64>(p, sp, stream);
 }
 
 }  // namespace
@@ -604,19 +676,25 @@ bool prefill_mfma_supported(DType dt, int head_dim, int block_size) {
          block_size >= 512 / head_dim;
 }
 
-// One workgroup per item only.
-PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &) { return {kRows, 0}; }
-
-hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *,
-                               hipStream_t stream) {
-  // The tile loader computes addresses inside a block with 32-bit byte
-  // offsets below 2^31; pools with larger blocks take the VALU kernel.
+// The tile loader computes addresses inside a block with 32-bit byte offsets
+// below 2^31; pools with larger blocks, and groups of more query heads than a
+// workgroup has rows, take the VALU kernel.
+static bool mfma_covers(const PrefillParams &p) {
   const uint64_t eb = 2, lim = (uint64_t)1 << 31;
-  const bool narrow = (uint64_t)p.kv_stride_block * eb < lim &&
-                      ((uint64_t)p.kv_stride_token * eb << p.block_shift) < lim;
-  if (p.group > kRows || !narrow) return launch_prefill_valu(p, dt, stream);
-  if (dt == DType::BF16) return launch_t<__bf16>(p, stream);
-  if (dt == DType::F16) return launch_t<_Float16>(p, stream);
+  return p.group <= kRows && (uint64_t)p.kv_stride_block * eb < lim &&
+         ((uint64_t)p.kv_stride_token * eb << p.block_shift) < lim;
+}
+
+PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &p) {
+  if (!mfma_covers(p)) return {kRows, 0};
+  return prefill_split_shape(p, kRows, kBK, 1, 4, kSplitMinTiles, true);
+}
+
+hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *sp,
+                               hipStream_t stream) {
+  if (!mfma_covers(p)) return launch_prefill_valu(p, dt, stream);
+  if (dt == DType::BF16) return launch_t<__bf16>(p, sp, stream);
+  if (dt == DType::F16) return launch_t<_Float16>(p, sp, stream);
   return hipErrorInvalidValue;
 }
 

@@ -36,6 +36,7 @@ LENS = [([0], [511]), ([2000], [1]), ([31, 32, 33, 63, 64, 65], [33, 32, 31, 1, 
 @pytest.mark.parametrize("lens", range(len(LENS)))
 @pytest.mark.parametrize("hq,hkv,d,bs,dtype", [
     (12, 12, 64, 16, torch.float32), (28, 4, 128, 16, torch.float32), (64, 1, 128, 4, torch.float32),
+    (28, 4, 128, 16, torch.bfloat16), (12, 12, 64, 32, torch.bfloat16), (8, 8, 128, 16, torch.float16),
 ])
 def test_split_prefill_matches_oracle(lens, hq, hkv, d, bs, dtype):
     cached, new = LENS[lens]
@@ -80,7 +81,7 @@ def native_call(q, k, v, tables, ctx, qsl, max_q, scale, split):
     return out.cpu()
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("scale", [0.1, -0.1, 0.0])
 def test_split_equals_whole(dtype, scale):
     """Same outputs as one workgroup per item: short contexts (fewer cached
