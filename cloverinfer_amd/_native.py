@@ -224,10 +224,10 @@ _host_tried = False
 
 
 def load_host():
-    """The node backend's native payload gather (cloverinfer_amd/_lib/_clv_host.so,
+    """The Python layer's native host code (cloverinfer_amd/_lib/_clv_host.so,
     built by cloverinfer_amd/build.py), or None when it is absent or does not
     load: it is host plumbing, and the backend then stages payloads with
-    torch.stack."""
+    torch.stack and kernels.py fills argument blocks in Python."""
     global _host, _host_tried
     if _host_tried:
         return _host

@@ -47,10 +47,11 @@ SOURCES = [
 
 ARCH = "gfx950"
 
-# The node backend's native payload gather (a Python extension on torch's C++
-# API, host code only; cloverinfer_amd/host/node_gather.cpp).
+# The Python layer's native host code (an extension on torch's C++ API): the
+# node backend's payload gather (host/node_gather.cpp) and the argument blocks
+# of the C ABI from tensors (host/call_args.cpp).
 HOST_EXT_NAME = "_clv_host"
-HOST_EXT_SRC = os.path.join(PKG_DIR, "host", "node_gather.cpp")
+HOST_EXT_SRCS = [os.path.join(PKG_DIR, "host", f) for f in ("node_gather.cpp", "call_args.cpp")]
 HOST_EXT_PATH = os.path.join(LIB_DIR, HOST_EXT_NAME + ".so")
 
 SANITIZE_LIB_PATH = os.path.join(LIB_DIR, "sanitize", LIB_NAME)
@@ -142,19 +143,19 @@ def build_host_ext(verbose: bool = False) -> str:
 
     os.makedirs(LIB_DIR, exist_ok=True)
     inc = [f for p in ce.include_paths() for f in ("-I", p)]
-    inc += ["-I", sysconfig.get_paths()["include"]]
+    inc += ["-I", INCLUDE_DIR, "-I", sysconfig.get_paths()["include"]]
     lib = ce.library_paths()[0]
     tmp = HOST_EXT_PATH + ".tmp"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fopenmp", *inc,
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-DTORCH_EXTENSION_NAME={HOST_EXT_NAME}", "-DTORCH_API_INCLUDE_EXTENSION_H",
-           HOST_EXT_SRC, "-o", tmp, f"-L{lib}", "-lc10", "-ltorch", "-ltorch_cpu",
+           *HOST_EXT_SRCS, "-o", tmp, f"-L{lib}", "-lc10", "-ltorch", "-ltorch_cpu",
            "-ltorch_python", f"-Wl,-rpath,{lib}"]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"g++ failed for {HOST_EXT_SRC}:\n{res.stderr[-4000:]}")
+        raise RuntimeError(f"g++ failed for {HOST_EXT_SRCS}:\n{res.stderr[-4000:]}")
     os.replace(tmp, HOST_EXT_PATH)
     return HOST_EXT_PATH
 

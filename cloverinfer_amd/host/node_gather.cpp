@@ -12,6 +12,8 @@
 // tensor and copies the rows with a parallel memcpy. It is host plumbing of
 // the Python backend (torch types are fine here); the paged-attention C ABI
 // (include/clover_attn.h) does not depend on it.
+#include "call_args.h"
+
 #include <torch/extension.h>
 
 #include <ATen/Parallel.h>
@@ -153,4 +155,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gather_rows", &gather_rows, "copy a list of CPU tensors into the rows of dst");
   m.def("copy_rows", &copy_rows, "copy a contiguous CPU tensor into dst in parallel");
   m.def("parse_batch", &parse_batch, "one pass over a uniform decode batch of item dicts");
+  m.def("fill_decode_args", &clv_host::fill_decode_args, "clv_decode_args from tensors");
+  m.def("fill_prefill_args", &clv_host::fill_prefill_args, "clv_prefill_args from tensors");
+  m.def("fill_cache_args", &clv_host::fill_cache_args, "clv_cache_args from tensors");
 }

@@ -8,6 +8,7 @@ call goes through ``libclover_attn.so``; tensors must live on a HIP device.
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 import threading
@@ -77,8 +78,28 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+# The current stream's handle without building a torch.cuda.Stream around it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _filled(name: str, args, *values):
+    """``args`` (an argument block of the C ABI) filled from a call's tensors
+    by the native host code, or None where that is absent or does not take
+    them as they are (the Python checks then raise, or fill it themselves)."""
+    host = _native.load_host()
+    fill = getattr(host, name, None)
+    if fill is None:
+        return None
+    try:
+        return args if fill(ctypes.addressof(args), *values) else None
+    except TypeError:  # a number given as something else than an int
+        return None
 
 
 def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
@@ -148,6 +169,11 @@ def _workspace_reused(ws: torch.Tensor, key, epoch: int) -> bool:
 
 def _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                  max_context_len, scale) -> _native.DecodeArgs:
+    a = _filled("fill_decode_args", _native.DecodeArgs(), out, q, k_cache, v_cache, block_tables,
+                context_lens, block_size, max_context_len, scale)
+    if a is not None:
+        return a
+    _require_device(out, q, k_cache, v_cache, block_tables, context_lens)
     if q.dim() != 3 or out.shape != q.shape:
         raise ValueError("q and out must both be [num_seqs, num_heads, head_dim]")
     _check_cache(k_cache, v_cache)
@@ -200,7 +226,6 @@ def decode_args(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                 scale: float | None = None) -> _native.DecodeArgs:
     """Validated C-ABI argument block of a paged decode (tensors stay owned
     by the caller and must outlive every launch made with it)."""
-    _require_device(out, q, k_cache, v_cache, block_tables, context_lens)
     return _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                         max_context_len, scale)
 
@@ -256,9 +281,9 @@ def paged_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     ``v_scale`` (numbers or per-kv-head values), balanced schedule only
     (head_dim 128, block_size >= 16), ``partition_size`` must be None.
     """
-    dev = _require_device(out, q, k_cache, v_cache, block_tables, context_lens)
     a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                      max_context_len, scale)
+    dev = q.device
     lib = _native.load()
     stream = _stream(dev)
     if k_cache.dtype == FP8:
@@ -308,10 +333,9 @@ class AppendDecodeLaunch:
                  v_cache: torch.Tensor, block_tables: torch.Tensor, context_lens: torch.Tensor,
                  block_size: int, max_context_len: int, key_new: torch.Tensor,
                  value_new: torch.Tensor, scale: float | None = None, num_waves: int = 0):
-        self.device = _require_device(out, q, k_cache, v_cache, block_tables, context_lens,
-                                      key_new, value_new)
         a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                          max_context_len, scale)
+        self.device = _require_device(q, key_new, value_new)
         if not balanced_supported(a):
             raise NotImplementedError("paged_attention_append covers the balanced decode's shapes only")
         shape = (a.num_seqs, a.num_kv_heads, a.head_dim)
@@ -412,9 +436,9 @@ class SplitAppendDecode:
                  v_cache: torch.Tensor, block_tables: torch.Tensor, context_lens: torch.Tensor,
                  block_size: int, max_context_len: int, scale: float | None = None,
                  num_waves: int = 0):
-        self.device = _require_device(out, q, k_cache, v_cache, block_tables, context_lens)
         a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                          max_context_len, scale)
+        self.device = q.device
         if not balanced_supported(a):
             raise NotImplementedError("the split decode covers the balanced decode's shapes only")
         self.args = a
@@ -568,6 +592,10 @@ def splitk_reduce(a: _native.DecodeArgs, partition_size: int, workspace: torch.T
 
 
 def _cache_args(key, value, k_cache, v_cache, slot_mapping) -> _native.CacheArgs:
+    a = _filled("fill_cache_args", _native.CacheArgs(), key, value, k_cache, v_cache, slot_mapping)
+    if a is not None:
+        return a
+    _require_device(key, value, k_cache, v_cache, slot_mapping)
     _check_cache(k_cache, v_cache)
     num_blocks, bs, num_kv_heads, head_dim = k_cache.shape
     if key.dim() != 3 or value.shape != key.shape or key.shape[1:] != (num_kv_heads, head_dim):
@@ -615,8 +643,8 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Ten
     ``slot_mapping[i]`` (= block*block_size + offset; negative slots are skipped).
     fp8 pools store e4m3(clamp(x / scale, -448, 448)) with per-kv-head
     ``k_scale``/``v_scale``."""
-    dev = _require_device(key, value, k_cache, v_cache, slot_mapping)
     a = _cache_args(key, value, k_cache, v_cache, slot_mapping)
+    dev = k_cache.device
     if k_cache.dtype == FP8:
         num_kv_heads = k_cache.shape[2]
         ks = kv_scales(k_scale, num_kv_heads, dev)
@@ -628,21 +656,9 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Ten
     _native.check(_native.load().clv_reshape_and_cache(a, _stream(dev)), "clv_reshape_and_cache")
 
 
-def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
-                    v_cache: torch.Tensor, block_tables: torch.Tensor,
-                    context_lens: torch.Tensor, query_start_loc: torch.Tensor,
-                    max_query_len: int | None, scale: float | None = None) -> None:
-    """Causal attention of each sequence's new query rows over its paged context.
-
-    Sequence s owns rows ``query_start_loc[s]:query_start_loc[s+1]`` of q/out;
-    its new tokens are the last ones of its ``context_lens[s]`` cached tokens,
-    and row i sees positions ``<= context_lens[s] - n_s + i``.
-    ``max_query_len`` must be at least every chunk length n_s (it sizes the
-    launch; a row i >= max_query_len of its chunk comes out as NaN, in every
-    kernel form); None computes it from ``query_start_loc`` with one small
-    device-to-host copy.
-    """
-    dev = _require_device(out, q, k_cache, v_cache, block_tables, context_lens, query_start_loc)
+def _prefill_args(out, q, k_cache, v_cache, block_tables, context_lens, query_start_loc,
+                  max_query_len, scale) -> _native.PrefillArgs:
+    _require_device(out, q, k_cache, v_cache, block_tables, context_lens, query_start_loc)
     _check_cache(k_cache, v_cache)
     if q.dim() != 3 or out.shape != q.shape:
         raise ValueError("q and out must both be [num_tokens, num_heads, head_dim]")
@@ -685,6 +701,31 @@ def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     a.num_blocks = num_blocks
     a.dtype = _dtype_code(q)
     a.scale = float(scale)
+    return a
+
+
+def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
+                    v_cache: torch.Tensor, block_tables: torch.Tensor,
+                    context_lens: torch.Tensor, query_start_loc: torch.Tensor,
+                    max_query_len: int | None, scale: float | None = None) -> None:
+    """Causal attention of each sequence's new query rows over its paged context.
+
+    Sequence s owns rows ``query_start_loc[s]:query_start_loc[s+1]`` of q/out;
+    its new tokens are the last ones of its ``context_lens[s]`` cached tokens,
+    and row i sees positions ``<= context_lens[s] - n_s + i``.
+    ``max_query_len`` must be at least every chunk length n_s (it sizes the
+    launch; a row i >= max_query_len of its chunk comes out as NaN, in every
+    kernel form); None computes it from ``query_start_loc`` with one small
+    device-to-host copy.
+    """
+    a = None
+    if max_query_len is not None:
+        a = _filled("fill_prefill_args", _native.PrefillArgs(), out, q, k_cache, v_cache,
+                    block_tables, context_lens, query_start_loc, max_query_len, scale)
+    if a is None:
+        a = _prefill_args(out, q, k_cache, v_cache, block_tables, context_lens, query_start_loc,
+                          max_query_len, scale)
+    dev = q.device
     lib = _native.load()
     nbytes = lib.clv_prefill_workspace_bytes(a)
     if nbytes:
