@@ -744,7 +744,7 @@ clv::PrefillSplitShape split_shape(const clv::PrefillParams &p, PrefillKernel k)
 
 size_t split_bytes(const clv::PrefillParams &p, const clv::PrefillSplitShape &sh) {
   const size_t rows = 2 * (size_t)sh.groups * (size_t)sh.rows;
-  return round256((size_t)sh.groups * 16) + 2 * round256(rows * 4) +
+  return round256((size_t)sh.groups * clv::kPrefillDescBytes) + 2 * round256(rows * 4) +
          round256(rows * (size_t)p.head_dim * 4);
 }
 
@@ -820,8 +820,8 @@ int clv_chunked_prefill_split(const clv_prefill_args *a, void *workspace, size_t
   char *ws = (char *)workspace;
   clv::PrefillSplit sp;
   sp.groups = sh.groups;
-  sp.desc = (int32_t *)ws;
-  ws += round256((size_t)sh.groups * 16);
+  sp.desc = ws;
+  ws += round256((size_t)sh.groups * clv::kPrefillDescBytes);
   sp.ws_m = (float *)ws;
   ws += round256(rows * 4);
   sp.ws_l = (float *)ws;

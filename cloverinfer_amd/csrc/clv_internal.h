@@ -104,13 +104,15 @@ struct PrefillParams {
   int32_t cus_per_xcd;
 };
 
+constexpr int kPrefillDescBytes = 32;
+
 // Workspace of a split prefill (prefill_split.h): one descriptor per group
 // and two partials of `rows` rows each.
 struct PrefillSplit {
   float *ws_o;    // [2 * groups, rows, head_dim] unnormalised contexts
   float *ws_m;    // [2 * groups, rows] row max of the unscaled scores
   float *ws_l;    // [2 * groups, rows] row sum
-  int32_t *desc;  // [groups, 4]
+  void *desc;     // [groups] descriptors of kPrefillDescBytes
   int32_t groups;
 };
 

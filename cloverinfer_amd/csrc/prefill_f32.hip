@@ -38,11 +38,11 @@ constexpr int kRows = kWaves * 16;  // query rows per workgroup
 constexpr int kBK = 32;             // K/V tokens per tile
 static_assert(kWaves == 4, "the per-wave flags are read as one word");
 
-// Workgroups (and so waves per SIMD) of a compute unit. More of them at
-// head_dim 64 hide more latency but cut the items into more partials: 8 x 512
-// tokens, 12 heads: 68.7 us at two, 64.2 at three, 85.8 at four; one sequence
-// of 512: 27.1, 32.8 and 46.2 us.
-constexpr int kPerCu = 2;
+// Workgroups (and so waves per SIMD) of a compute unit: what the registers
+// allow. At head_dim 64 (162 VGPRs) three against two: 8 x 512 tokens, 12 heads
+// 69.8 -> 65.1 us, 4 x 512 over 2048 cached 210 -> 192, one prompt of 512
+// 26.2 -> 25.8; four (128 VGPRs, spilled) 85 us on the first.
+constexpr int per_cu(int head_dim) { return head_dim == 64 ? 3 : 2; }
 
 struct SplitCfg {
   static constexpr int kBK = clv::kBK;
@@ -62,7 +62,7 @@ __device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {
 constexpr int kSplitMinTiles = 6;
 
 template <int D, bool SPLIT>
-__global__ void __launch_bounds__(kThreads, kPerCu)
+__global__ void __launch_bounds__(kThreads, per_cu(D))
 chunked_prefill_f32(const PrefillArgs args) {
   constexpr int NQK = D / 16;            // 16-byte Q / K words per lane
   constexpr int CH = D / 16;             // output blocks
@@ -89,14 +89,16 @@ chunked_prefill_f32(const PrefillArgs args) {
   // contiguous range of logical work, so that the query tiles of one kv head
   // share its L2.
   const int per_xcd = gridDim.x / 8;
-  const int L = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  int L = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
 
   typedef PrefillSched<SplitCfg> Sched;
   if constexpr (SPLIT) {
     Sched sched;
     sched.init<kThreads>(args.p, args.bq, args.n_qtiles, args.sp.groups, s_pre, s_tmp);
+    L = sched.group_of(blockIdx.x);
+    if (L < 0) return;
     sched.start(L, s_cur[wave]);
-    if (tid == 0) reinterpret_cast<PrefillDesc *>(args.sp.desc)[L] = PrefillDesc{-1, 0, 0, 0};
+    if (tid == 0) sched.clear_desc(args.sp, L);
   } else if (L >= args.total) {
     return;
   }
@@ -361,7 +363,7 @@ chunked_prefill_f32(const PrefillArgs args) {
     const int64_t prow = (int64_t)(2 * L + (t0 == 0 ? 1 : 0)) * kRows;  // partial's first row
     if constexpr (SPLIT) {
       if (!whole) {
-        if (tid == 0) prefill_note(ar1.sp, L, it, t0 == 0, t1 == nt);
+        if (tid == 0) prefill_note(ar1.sp, L, it, G, t0 == 0, t1 == nt);
         if (j == 0 && 16 * wave + n16 < rows) {
           ar1.sp.ws_m[prow + 16 * wave + n16] = m_run;
           ar1.sp.ws_l[prow + 16 * wave + n16] = l_run;
@@ -431,7 +433,7 @@ bool prefill_f32_supported(const PrefillParams &p, int block_size) {
 }
 
 PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p) {
-  return prefill_split_shape(p, kRows, kBK, kPerCu, 1, kSplitMinTiles, false);
+  return prefill_split_shape(p, kRows, kBK, per_cu(p.head_dim), 1, kSplitMinTiles, false);
 }
 
 hipError_t launch_prefill_f32(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream) {

@@ -162,17 +162,17 @@ chunked_prefill_mfma(const PrefillArgs args) {
   // dispatch_slot sets.
   const int per_xcd = gridDim.x / 8;
   const int xcd0 = (blockIdx.x % 8) * per_xcd;
-  const int L = SPLIT ? xcd0 + blockIdx.x / 8
-                      : xcd0 + dispatch_slot(blockIdx.x / 8, per_xcd, args.total - xcd0,
+  int L = SPLIT ? 0 : xcd0 + dispatch_slot(blockIdx.x / 8, per_xcd, args.total - xcd0,
                                              args.n_qtiles, args.p.cus_per_xcd);
   typedef PrefillSched<SplitCfg> Sched;
   int *cur = s_cur[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
   if constexpr (SPLIT) {
     Sched sched;
     sched.init<kThreads>(args.p, args.bq, args.n_qtiles, args.sp.groups, s_pre, s_tmp);
+    L = sched.group_of(blockIdx.x);
+    if (L < 0) return;
     sched.start(L, cur);
-    if (threadIdx.x == 0)
-      reinterpret_cast<PrefillDesc *>(args.sp.desc)[L] = PrefillDesc{-1, 0, 0, 0};
+    if (threadIdx.x == 0) sched.clear_desc(args.sp, L);
   } else if (L >= args.total) {
     return;
   }
@@ -602,7 +602,7 @@ chunked_prefill_mfma(const PrefillArgs args) {
   const PrefillArgs ar1 = SPLIT ? reload_args() : args;
   const bool whole = !SPLIT || (t0 == 0 && t1 == nt);
   const int64_t prow = (int64_t)(2 * L + (t0 == 0 ? 1 : 0)) * kRows;
-  if (SPLIT && !whole && tid == 0) prefill_note(ar1.sp, L, it, t0 == 0, t1 == nt);
+  if (SPLIT && !whole && tid == 0) prefill_note(ar1.sp, L, it, G, t0 == 0, t1 == nt);
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
     if (SPLIT && !whole && j == 0)

@@ -30,12 +30,18 @@
 namespace clv {
 
 // What a group left in the workspace: the item whose first part it holds
-// (s < 0: none; partial slot 2w + 1), and whether its first item was begun
-// by an earlier group (cont, partial slot 2w) and ends here.
+// (rows 0: none; partial slot 2w + 1), and whether its first item was begun
+// by an earlier group (cont, partial slot 2w) and ends here. The item is
+// described by what the merge needs, so that it reads nothing else first.
 struct __attribute__((aligned(16))) PrefillDesc {
-  int32_t s, kvh, qt;
+  int32_t rows;  // query rows of the item (tokens x query heads)
+  int32_t row0;  // token row of q / out of its first token
+  int32_t q0;    // that token's index in its chunk
+  int32_t kvh;
   int32_t cont;  // 0: none, 1: goes on in the next group, 2: ends here
+  int32_t unused[3];
 };
+static_assert(sizeof(PrefillDesc) == kPrefillDescBytes, "the workspace layout");
 
 // One work item.
 struct PrefillItem {
@@ -151,8 +157,23 @@ struct PrefillSched {
     __syncthreads();
     C = __builtin_amdgcn_readfirstlane(whole ? tc : tu);
     N = C * H;
-    W = whole ? N : min(groups, max(1, N / Cfg::kMinShare));
+    W = whole ? max(1, N) : min(groups, max(1, N / Cfg::kMinShare));
     tol = whole ? 0 : Cfg::snap(share);
+  }
+
+  // Group of workgroup `block`, or -1. Consecutive ids go round-robin over the
+  // 8 XCDs: each takes a contiguous run of the W groups in use (query tiles of
+  // one kv head then share its L2), the idle workgroups spread over all of them.
+  __device__ __forceinline__ int group_of(int block) const {
+    const int per_xcd = (W + 7) / 8;
+    const int w = (block % 8) * per_xcd + block / 8;
+    return block / 8 < per_xcd && w < W ? w : -1;
+  }
+
+  // Clears the descriptor of group w, and those past W between all groups.
+  __device__ __forceinline__ void clear_desc(const PrefillSplit &sp, int w) const {
+    for (int i = w; i < sp.groups; i += W)
+      reinterpret_cast<PrefillDesc *>(sp.desc)[i] = PrefillDesc{0, 0, 0, 0, 0, {0, 0, 0}};
   }
 
   // Entry holding unit rem of a kv head (0 <= rem < C): the last one with
@@ -258,59 +279,68 @@ __device__ __forceinline__ PrefillArgs reload_args() {
 // Records the partial that group w leaves of item `it`: its first part, or a
 // later one that ends the item or not. One thread writes all of a group's.
 __device__ __forceinline__ void prefill_note(const PrefillSplit &sp, int w, const PrefillItem &it,
-                                             bool begins, bool ends) {
+                                             int group, bool begins, bool ends) {
   PrefillDesc *d = reinterpret_cast<PrefillDesc *>(sp.desc) + w;
   if (begins) {
-    d->s = it.s;
+    d->rows = (it.q_hi - it.q0) * group;
+    d->row0 = it.qs + it.q0;
+    d->q0 = it.q0;
     d->kvh = it.kvh;
-    d->qt = it.qt;
   } else {
     d->cont = ends ? 2 : 1;
   }
 }
 
 // Merges the partials of the items that the split cut: workgroup (w, y)
-// takes rows [y * kMergeRows, ..) of the item that group w begins and does
-// not finish. Bound by the partials' bytes; LPR lanes share a row (16 bytes
-// each), lane k of them weighs partial k, so that weights cost one round trip
-// for up to LPR partials.
+// takes rows [y * kPrefillMergeRows, ..) of the item that group w begins and
+// does not finish. Bound by memory latency for a few partials, by their bytes
+// for many; so the descriptors of w and of the groups after it are read
+// together, then the weights and contexts of a row's first four partials.
+// LPR lanes share a row (16 bytes each), lane k of them weighs partial k.
 constexpr int kPrefillMergeRows = 32;
 
 template <typename T, int D, int ROWS>
 __global__ void __launch_bounds__(256)
 prefill_merge(const PrefillArgs args) {
-  const PrefillParams &p = args.p;
-  const PrefillSplit &sp = args.sp;
-  const int bq = args.bq;
   constexpr int LPR = D / 4;
   constexpr int RPP = 256 / LPR;
-  static_assert(ROWS % kPrefillMergeRows == 0 || ROWS < kPrefillMergeRows, "row chunks");
+  static_assert(ROWS % kPrefillMergeRows == 0, "row chunks");
+  const PrefillParams &p = args.p;
+  const PrefillSplit &sp = args.sp;
   const PrefillDesc *desc = (const PrefillDesc *)sp.desc;
   const int w = blockIdx.x;
-  const PrefillDesc d = desc[w];
-  if (d.s < 0) return;
   const int lane = threadIdx.x & 63;
+  const int32_t cont0 = desc[min(w + 1 + lane, sp.groups - 1)].cont;
+  const PrefillDesc d = desc[w];
+  const int r_end = min(d.rows, (int)(blockIdx.y + 1) * kPrefillMergeRows);
+  if ((int)blockIdx.y * kPrefillMergeRows >= r_end) return;
   int n = 1;
   for (int b = w + 1; b < sp.groups; b += 64) {
-    const uint64_t ends = __ballot(b + lane < sp.groups && desc[b + lane].cont == 2);
+    const int32_t c = b == w + 1 ? cont0 : desc[min(b + lane, sp.groups - 1)].cont;
+    const uint64_t ends = __ballot(b + lane < sp.groups && c == 2);
     if (ends != 0) {
       n = b - w + __builtin_ctzll(ends) + 1;
       break;
     }
   }
-  PrefillItem it;
-  it.set(p, bq, d.s, d.kvh, d.qt);
   const int G = p.group;
-  const int rows = (it.q_hi - it.q0) * G;
   const int sub = threadIdx.x % LPR;
-  const int r_end = min(rows, (int)(blockIdx.y + 1) * kPrefillMergeRows);
+  const float c = fmaxf(fabsf(p.scale_log2), 0x1p-126f);  // as the kernels scale scores
   for (int r = blockIdx.y * kPrefillMergeRows + threadIdx.x / LPR; r < r_end; r += RPP) {
     auto row_of = [&](int k) {  // row of partial k in the workspace
       return (int64_t)(k == 0 ? 2 * w + 1 : 2 * (w + k)) * ROWS + r;
     };
-    const float c = fmaxf(fabsf(p.scale_log2), 0x1p-126f);  // as the kernels scale scores
-    float M = kNegInf;
-    for (int k = sub; k < n; k += LPR) M = fmaxf(M, sp.ws_m[row_of(k)]);
+    auto load4 = [&](int k0, f32x4 (&v)[4]) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = load_vec<f32x4>(sp.ws_o + row_of(min(k0 + u, n - 1)) * D + 4 * sub);
+    };
+    const float m0 = sub < n ? sp.ws_m[row_of(sub)] : kNegInf;
+    const float l0 = sub < n ? sp.ws_l[row_of(sub)] : 0.f;
+    f32x4 v[4];
+    load4(0, v);
+    float M = m0;
+    for (int k = sub + LPR; k < n; k += LPR) M = fmaxf(M, sp.ws_m[row_of(k)]);
 #pragma unroll
     for (int off = 1; off < LPR; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, LPR));
     const float Msub = M == kNegInf ? 0.f : M;
@@ -320,14 +350,11 @@ prefill_merge(const PrefillArgs args) {
       const int cnt = min(LPR, n - k0);
       float wk = 0.f;
       if (sub < cnt) {
-        wk = fast_exp2((sp.ws_m[row_of(k0 + sub)] - Msub) * c);
-        L += sp.ws_l[row_of(k0 + sub)] * wk;
+        wk = fast_exp2(((k0 == 0 ? m0 : sp.ws_m[row_of(k0 + sub)]) - Msub) * c);
+        L += (k0 == 0 ? l0 : sp.ws_l[row_of(k0 + sub)]) * wk;
       }
       for (int k = 0; k < cnt; k += 4) {  // four rows' loads in flight
-        f32x4 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          v[u] = load_vec<f32x4>(sp.ws_o + row_of(k0 + min(k + u, cnt - 1)) * D + 4 * sub);
+        if (k0 + k > 0) load4(k0 + k, v);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const float f = __shfl(wk, min(k + u, LPR - 1), LPR);
@@ -337,9 +364,10 @@ prefill_merge(const PrefillArgs args) {
     }
 #pragma unroll
     for (int off = 1; off < LPR; off <<= 1) L += __shfl_xor(L, off, LPR);
-    const int tok = it.q0 + r / G;
-    const float inv = tok >= p.max_query_len ? __builtin_nanf("") : L > 0.f ? 1.f / L : 0.f;
-    T *dst = (T *)p.out + (int64_t)(it.qs + tok) * p.out_stride_token +
+    const int tok = r / G;
+    const float inv =
+        d.q0 + tok >= p.max_query_len ? __builtin_nanf("") : L > 0.f ? 1.f / L : 0.f;
+    T *dst = (T *)p.out + (int64_t)(d.row0 + tok) * p.out_stride_token +
              (int64_t)(d.kvh * G + r % G) * p.out_stride_head + 4 * sub;
     if constexpr (sizeof(T) == 4) {
       store_vec<f32x4>(dst, acc * inv);
