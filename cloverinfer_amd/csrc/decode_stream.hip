@@ -151,7 +151,7 @@ __device__ int block_exclusive_scan(int *buf, int n, int *tmp) {
   return total;
 }
 
-// APPEND (K-transpose path only): fused append, see below.
+// APPEND (UNI only): fused append, see below.
 // KV8 (K-transpose path only): fp8 pools, see DecodeWave.
 // PART: split-K partials (partition_size > 0). The unit of the split is a
 // partition of partition_size tokens instead of a 16-token step (no phantom
@@ -238,34 +238,6 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
   w.init(p);
   w.set_k_lds(s_kt[uni(threadIdx.x >> 6)]);
 
-  if constexpr (APPEND) {
-    // Fused append: the wave that holds a segment's last step writes the
-    // sequence's new token (position ctx - 1) before its run loop. Only that
-    // wave ever loads the row (one query-head chunk per kv head on this
-    // path), with the lanes that wrote it (kt_store_row).
-    static_assert(UNI && D == 128, "the fused append mirrors the K-transpose loads");
-    for (int sg = seg; sg < nseg && uni(s_seg[sg + 1]) - 1 < en; ++sg) {
-      const int lst = uni(s_seg[sg + 1]) - 1;
-      if (lst < st || lst < uni(s_seg[sg]) + K) continue;  // not ours, or no real steps
-      const int s_ = sg / per_seq;
-      const int kvh = (sg - s_ * per_seq) * HG + wk;  // one query-head chunk per kv head
-      const int ctx = clamp_ctx(p, lens, s_);
-      if (ctx != scalar_load_i32(lens + s_)) continue;  // the new position is not attended
-      const SegGeom geo = seg_geom<T>(p, s_, kvh, ctx, tables);
-      const int pos = ctx - 1;
-      const int blk = scalar_load_i32(geo.bt + (pos >> p.block_shift));
-      if ((unsigned)blk >= (unsigned)p.num_blocks) continue;
-      const int64_t row_off =
-          ((int64_t)blk * p.kv_stride_block + (int64_t)(pos & ((1 << p.block_shift) - 1)) *
-                                                  p.kv_stride_token) * (int64_t)sizeof(T);
-      const int64_t src = (int64_t)s_ * p.new_stride_seq + (int64_t)kvh * p.new_stride_head;
-      kt_store_row(geo.kbase, geo.vbase, row_off, pos,
-                   (const uint16_t *)p.key_new + src, (const uint16_t *)p.value_new + src);
-    }
-    __builtin_amdgcn_s_waitcnt(0);      // the stores are done before any load is issued
-    __asm__ volatile("" ::: "memory");  // and the compiler keeps them ahead of the loads
-  }
-
   // The span is cut at segment borders into runs. Each run loads its Q rows,
   // keeps DEPTH steps of loads in flight (a ring of register sets refilled
   // right after each step is folded) and ends with one partial.
@@ -331,6 +303,30 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
     };
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) issue(xs + i, R[i]);
+    // Fused append: the run that holds a segment's last step has the
+    // sequence's new token (position ctx - 1) in that step, and only its wave
+    // loads that row (one query-head chunk per kv head on this path). The row
+    // as loaded from the pool is replaced in registers before the step is
+    // folded, and the new row is written when the run has ended, so the append
+    // adds no round trip to the wave (written before the ring and loaded back,
+    // it added as much as an append launch of its own). The loads are
+    // unconditional: a branch around them would make the compiler wait for
+    // every load in flight.
+    typename WV::NewRow nr;
+    bool append = false;
+    int64_t new_off = 0;
+    if constexpr (APPEND) {
+      static_assert(UNI, "the new row replaces one row of a step in one block");
+      const int64_t src = (int64_t)s_ * p.new_stride_seq + (int64_t)kvh * p.new_stride_head;
+      w.load_new((const T *)p.key_new + src, (const T *)p.value_new + src, nr);
+      const int nblk = brow[(ctx - 1) >> p.block_shift];
+      // A context past what the table covers does not attend its new position.
+      append = last == uni(s_seg[seg + 1]) - 1 && ctx == scalar_load_i32(lens + s_) &&
+               (unsigned)nblk < (unsigned)p.num_blocks;
+      new_off = ((int64_t)nblk * p.kv_stride_block +
+                 (int64_t)((ctx - 1) & ((1 << p.block_shift) - 1)) * p.kv_stride_token) *
+                (int64_t)sizeof(T);
+    }
     qk_t q[WV::NQK];
     w.mask_q(qraw, ng, q);
     int c = xs;
@@ -365,6 +361,9 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
 #pragma unroll
       for (int i = 0; i < DEPTH; ++i) {
         if (!done) {
+          if constexpr (APPEND) {
+            if (append && c == last) w.patch_row(ctx - 1, nr, R[i]);
+          }
           w.compute((c - first) * WV::STEP, ctx, R[i], q);
           if (++c > last)
             done = true;
@@ -400,6 +399,9 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
     // segment's partials at slot seg + (its first group) onwards.
     const int64_t row0 = (((int64_t)seg + wid) * HG + wk) * 16;
     w.store_partial(ws_o, ws_m, ws_l, row0, ng);
+    if constexpr (APPEND) {
+      if (append) w.store_new(geo.kbase, geo.vbase, new_off, ctx - 1, nr);
+    }
     w.reset();
     x = last + 1;
   }
@@ -536,13 +538,13 @@ hipError_t launch_stream_tdd(const DecodeParams &p, hipStream_t stream) {
                          p.seg_prefix);
       return hipGetLastError();
     }
-    if (p.append_new) {  // set only where stream_appends_in_kernel holds
-      if (p.block_shift < 4) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH, true>), grid, dim3(kThreads), 0,
-                         stream, p, p.block_tables, p.context_lens, p.ws_o, p.ws_m, p.ws_l,
-                         p.seg_prefix);
-      return hipGetLastError();
-    }
+  }
+  if (p.append_new) {  // set only where stream_appends_in_kernel holds
+    if (p.block_shift < 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH, true>), grid, dim3(kThreads), 0,
+                       stream, p, p.block_tables, p.context_lens, p.ws_o, p.ws_m, p.ws_l,
+                       p.seg_prefix);
+    return hipGetLastError();
   }
   if (p.block_shift >= 4)
     hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH>), grid, dim3(kThreads), 0, stream,
@@ -609,16 +611,20 @@ bool decode_stream_supported(DType dt, int head_dim, int block_size, int64_t num
 }
 
 bool stream_appends_in_kernel(DType dt, int head_dim, int block_size, int group) {
-  // The 16-bit K-transpose path (a 16-token step inside one block, head_dim
-  // 128) with one query-head chunk per kv head.
-  return (dt == DType::F16 || dt == DType::BF16) && head_dim == 128 && block_size >= 16 &&
-         group <= 16;
+  // A 16-token step inside one block, with one query-head chunk per kv head:
+  // then a single wave loads the appended row. Against an append launch of its
+  // own (fp32 and head_dim 64): 2 sequences of 1000..3000 tokens, 32/8 heads,
+  // fp32 23.9 -> 18.8 us a call (with the host's share), 16 of 500..1500, 12
+  // heads of 64, fp16 22.7 -> 19.7; 16 of 256..4096, 28/4 heads, fp32 33.8 ->
+  // 33.2, where the append ran beside the stream kernel's start.
+  return (dt == DType::F16 || dt == DType::BF16 || dt == DType::F32) &&
+         (head_dim == 64 || head_dim == 128) && block_size >= 16 && group <= 16;
 }
 
 hipError_t launch_decode_stream(const DecodeParams &p, DType dt, hipStream_t stream) {
   if (dt == DType::BF16) return launch_stream_t<__bf16>(p, stream);
   if (dt == DType::F16) return launch_stream_t<_Float16>(p, stream);
-  if (dt == DType::F32 && !p.kv_fp8 && !p.append_new) return launch_stream_t<float>(p, stream);
+  if (dt == DType::F32 && !p.kv_fp8) return launch_stream_t<float>(p, stream);
   return hipErrorInvalidValue;
 }
 
