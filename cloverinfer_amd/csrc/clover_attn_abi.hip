@@ -761,32 +761,6 @@ int launch_prefill(const clv::PrefillParams &p, DType dt, PrefillKernel k,
 
 }  // namespace
 
-namespace clv {
-
-PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
-                                      int tile_units, int min_tiles, bool even_rounds) {
-  const PrefillSplitShape none = {rows, 0};
-  const int64_t bq = rows / p.group;
-  const int64_t n_q = std::max<int64_t>(1, ceil_div(p.max_query_len, bq));
-  const int64_t max_tiles = ceil_div((int64_t)p.max_blocks_per_seq << p.block_shift, bk);
-  // The table width bounds every context: up to min_tiles tiles the longest
-  // item is short, and the split would cost its merge launch.
-  if (max_tiles <= min_tiles || p.cus_per_xcd <= 0) return none;
-  const int64_t entries = (int64_t)p.num_seqs * n_q;
-  if (entries > kPrefillSplitItems) return none;
-  // Units are 32-bit on the device (at most four of an item's own).
-  if (entries * p.num_kv_heads * (max_tiles + 4) * tile_units >= (int64_t)1 << 30) return none;
-  // Chunks of one length that fill whole rounds of the device: the 16-bit
-  // kernel's natural order (dispatch_slot) makes them even already.
-  const int groups = per_cu * p.cus_per_xcd * 8;
-  if (even_rounds && (int64_t)p.num_tokens == (int64_t)p.num_seqs * p.max_query_len &&
-      entries * p.num_kv_heads % groups == 0)
-    return none;
-  return {rows, groups};
-}
-
-}  // namespace clv
-
 extern "C" {
 
 int clv_chunked_prefill(const clv_prefill_args *a, clv_stream_t stream) {

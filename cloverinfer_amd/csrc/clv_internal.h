@@ -164,12 +164,6 @@ hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSp
 bool prefill_f32_supported(const PrefillParams &p, int block_size);
 PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p);
 hipError_t launch_prefill_f32(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream);
-// The decision behind the split shapes: `rows` query rows per workgroup, `bk`
-// K/V tokens per tile, `per_cu` workgroups per compute unit, at most
-// `tile_units` units per tile; no split up to `min_tiles` tiles, nor (with
-// `even_rounds`) of equal chunks that fill whole rounds of the device.
-PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
-                                      int tile_units, int min_tiles, bool even_rounds);
 hipError_t launch_prefill_valu(const PrefillParams &p, DType dt, hipStream_t stream);
 
 // Whether the MFMA decode kernel covers this shape/dtype.

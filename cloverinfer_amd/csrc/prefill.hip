@@ -8,9 +8,10 @@
 // 0..i one at a time (append-then-attend).
 //
 // This file holds the VALU form (any dtype; one workgroup per query row and
-// kv head). The MFMA form for fp16/bf16 is in prefill_mfma.hip. In both, a
-// row at index max_query_len or later of its chunk (a chunk longer than the
-// caller's max_query_len, a caller error) comes out as NaN.
+// kv head). The MFMA forms are in prefill_mfma.hip (fp16/bf16) and
+// prefill_f32.hip. In all of them a row at index max_query_len or later of its
+// chunk (a chunk longer than the caller's max_query_len, a caller error) comes
+// out as NaN.
 #include "attn_common.h"
 
 namespace clv {

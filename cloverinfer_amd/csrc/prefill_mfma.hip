@@ -48,7 +48,7 @@
 // Uneven batches run in the split form (prefill_split.h): a workgroup per
 // compute unit takes an even share of the items' tiles, cutting long items.
 // 24 sequences of 0..6000 cached tokens, 60 % of them bringing one token and
-// the rest up to 300 (28/4 heads, bf16): 357 -> 136 us. A wave without rows
+// the rest up to 300 (28/4 heads, bf16): 357 -> 117 us. A wave without rows
 // only stages tiles in either form (one prompt of 777 tokens, 32 heads, whose
 // last query tile has 9 of 256 rows: 36.4 -> 32.1 us).
 #include "prefill_split.h"
@@ -116,13 +116,19 @@ __host__ __device__ inline int dispatch_slot(int i, int per_xcd, int valid, int 
 }
 
 // Units of the split (prefill_split.h): a quarter of the time of a full tile.
+// A tile of few rows costs nearly as much as a full one (its loads are waited
+// for), an item's start two tiles. The mixed step described above: 138.4 us at
+// 2 units for up to 128 rows and 4 for the start, 122.7 at 3 and 4, 116.7 at 3
+// and 8 (114.1 at 4 and 8, which loses 9 % where one-token rows are 90 % of 24
+// sequences: 59.1 against 64.6 us); 141.6 and 218 where tiles of up to 32 rows
+// are priced at 2 and 1.
 struct SplitCfg {
   static constexpr int kBK = clv::kBK;
-  static constexpr int kItemUnits = 4;
+  static constexpr int kItemUnits = 8;
   static constexpr int kMinShare = 16;
   static constexpr int kCutUnits = 40;
-  static __device__ __forceinline__ int tile_units(int rows) { return rows > 128 ? 4 : 2; }
-  static __device__ __forceinline__ int snap(int share) { return max(4, share / 16); }
+  static __device__ __forceinline__ int tile_units(int rows) { return rows > 128 ? 4 : 3; }
+  static __device__ __forceinline__ int snap(int share) { return max(8, share / 16); }
 };
 
 // Tiles up to which no item is long enough for a cut to pay.

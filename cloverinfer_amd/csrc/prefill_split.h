@@ -25,9 +25,37 @@
 // its two partials and their merge) would cost more than the evenness gives.
 #pragma once
 
+#include <algorithm>
+
 #include "attn_common.h"
 
 namespace clv {
+
+// The decision behind the split shapes: `rows` query rows per workgroup, `bk`
+// K/V tokens per tile, `per_cu` workgroups per compute unit, at most
+// `tile_units` units per tile; no split up to `min_tiles` tiles, nor (with
+// `even_rounds`) of equal chunks that fill whole rounds of the device.
+inline PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
+                                      int tile_units, int min_tiles, bool even_rounds) {
+  const PrefillSplitShape none = {rows, 0};
+  const int64_t bq = rows / p.group;
+  const int64_t n_q = std::max<int64_t>(1, ((int64_t)p.max_query_len + bq - 1) / bq);
+  const int64_t max_tiles = (((int64_t)p.max_blocks_per_seq << p.block_shift) + bk - 1) / bk;
+  // The table width bounds every context: up to min_tiles tiles the longest
+  // item is short, and the split would cost its merge launch.
+  if (max_tiles <= min_tiles || p.cus_per_xcd <= 0) return none;
+  const int64_t entries = (int64_t)p.num_seqs * n_q;
+  if (entries > kPrefillSplitItems) return none;
+  // Units are 32-bit on the device (an item's own are at most four tiles').
+  if (entries * p.num_kv_heads * (max_tiles + 4) * tile_units >= (int64_t)1 << 30) return none;
+  // Chunks of one length that fill whole rounds of the device: the 16-bit
+  // kernel's natural order (dispatch_slot) makes them even already.
+  const int groups = per_cu * p.cus_per_xcd * 8;
+  if (even_rounds && (int64_t)p.num_tokens == (int64_t)p.num_seqs * p.max_query_len &&
+      entries * p.num_kv_heads % groups == 0)
+    return none;
+  return {rows, groups};
+}
 
 // What a group left in the workspace: the item whose first part it holds
 // (rows 0: none; partial slot 2w + 1), and whether its first item was begun

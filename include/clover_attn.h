@@ -340,7 +340,7 @@ int32_t clv_default_num_waves(void);
 int32_t clv_default_num_waves_fp8(void);
 
 /*
- * Chunked prefill over paged KV (MFMA for fp16/bf16). No counterpart in the
+ * Chunked prefill over paged KV. No counterpart in the
  * reference; defined as equal, row by row, to successive append-then-attend
  * decode steps of CpuAttentionBackend.decode_layer
  * (src/core/attention_backend.py:82-123).
