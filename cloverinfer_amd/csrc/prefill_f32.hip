@@ -418,7 +418,7 @@ hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t
     hipLaunchKernelGGL((chunked_prefill_f32<D, true>), dim3((unsigned)sp->groups), dim3(kThreads),
                        0, stream, args);
     hipLaunchKernelGGL((prefill_merge<float, D, kRows>),
-                       dim3((unsigned)sp->groups, kRows / kPrefillMergeRows), dim3(256), 0, stream,
+                       dim3((unsigned)sp->groups, kRows / merge_rows(kRows)), dim3(256), 0, stream,
                        args);
     return hipGetLastError();
   }

@@ -320,19 +320,25 @@ __device__ __forceinline__ void prefill_note(const PrefillSplit &sp, int w, cons
 }
 
 // Merges the partials of the items that the split cut: workgroup (w, y)
-// takes rows [y * kPrefillMergeRows, ..) of the item that group w begins and
+// takes rows [y * merge_rows(ROWS), ..) of the item that group w begins and
 // does not finish. Bound by memory latency for a few partials, by their bytes
 // for many; so the descriptors of w and of the groups after it are read
 // together, then the weights and contexts of a row's first four partials.
 // LPR lanes share a row (16 bytes each), lane k of them weighs partial k.
-constexpr int kPrefillMergeRows = 32;
+//
+// Rows of a workgroup: 16 of 256, so that one long item cut into many pieces
+// still fills the chip (64 rows over 4000 cached tokens, 28/4 heads, bf16: 40 us
+// a call against 52 at 32 rows and 54 at 64; the mixed step 115.5, 116.6 and
+// 115.8); 32 of the fp32 kernel's 64 (OPT-125m prompts 40.0 us, at 16 40.8).
+constexpr int merge_rows(int rows) { return rows > 64 ? 16 : 32; }
 
 template <typename T, int D, int ROWS>
 __global__ void __launch_bounds__(256)
 prefill_merge(const PrefillArgs args) {
   constexpr int LPR = D / 4;
   constexpr int RPP = 256 / LPR;
-  static_assert(ROWS % kPrefillMergeRows == 0, "row chunks");
+  constexpr int kChunk = merge_rows(ROWS);
+  static_assert(ROWS % kChunk == 0, "row chunks");
   const PrefillParams &p = args.p;
   const PrefillSplit &sp = args.sp;
   const PrefillDesc *desc = (const PrefillDesc *)sp.desc;
@@ -340,8 +346,8 @@ prefill_merge(const PrefillArgs args) {
   const int lane = threadIdx.x & 63;
   const int32_t cont0 = desc[min(w + 1 + lane, sp.groups - 1)].cont;
   const PrefillDesc d = desc[w];
-  const int r_end = min(d.rows, (int)(blockIdx.y + 1) * kPrefillMergeRows);
-  if ((int)blockIdx.y * kPrefillMergeRows >= r_end) return;
+  const int r_end = min(d.rows, (int)(blockIdx.y + 1) * kChunk);
+  if ((int)blockIdx.y * kChunk >= r_end) return;
   int n = 1;
   for (int b = w + 1; b < sp.groups; b += 64) {
     const int32_t c = b == w + 1 ? cont0 : desc[min(b + lane, sp.groups - 1)].cont;
@@ -354,7 +360,7 @@ prefill_merge(const PrefillArgs args) {
   const int G = p.group;
   const int sub = threadIdx.x % LPR;
   const float c = fmaxf(fabsf(p.scale_log2), 0x1p-126f);  // as the kernels scale scores
-  for (int r = blockIdx.y * kPrefillMergeRows + threadIdx.x / LPR; r < r_end; r += RPP) {
+  for (int r = blockIdx.y * kChunk + threadIdx.x / LPR; r < r_end; r += RPP) {
     auto row_of = [&](int k) {  // row of partial k in the workspace
       return (int64_t)(k == 0 ? 2 * w + 1 : 2 * (w + k)) * ROWS + r;
     };
