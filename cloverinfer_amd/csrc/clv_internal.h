@@ -52,7 +52,7 @@ struct DecodeParams {
   // Fused append (balanced mode): when append_new is set, sequence s's new
   // key/value rows key_new/value_new[s] ([num_kv_heads, head_dim], strides in
   // elements) are written at its context position context_lens[s] - 1 by the
-  // wave that computes that position, before it loads it.
+  // wave that computes that position, which attends them from registers.
   int32_t append_new;
   const void *key_new;
   const void *value_new;

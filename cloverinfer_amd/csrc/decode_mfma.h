@@ -232,49 +232,34 @@ struct DecodeWave {
 
   __device__ __forceinline__ void set_k_lds(char *buf) { k_lds = buf; }
 
-  // One token's new key/value rows, each lane's pieces in the layout of Regs
-  // (the K row or row chunk and the V chunk it holds of one row of a step).
+  // Fused append (K-transpose path): one token's new key/value rows, each
+  // lane's pieces in the layout of Regs (its chunk of the K and V row).
   struct NewRow {
-    u32x4 k[KT ? 1 : NQK];
+    u32x4 k;
     vchunk_t v;
   };
   __device__ __forceinline__ void load_new(const T *knew, const T *vnew, NewRow &nr) const {
-    if constexpr (KT) {
-      nr.k[0] = load_vec<u32x4>(knew + n16 * CH);
-    } else {
-#pragma unroll
-      for (int i = 0; i < NQK; ++i) nr.k[i] = load_vec<u32x4>(knew + 32 * i + 8 * j);
-    }
+    static_assert(KT, "the fused append mirrors the K-transpose loads");
+    nr.k = load_vec<u32x4>(knew + n16 * CH);
     nr.v = load_vec<vchunk_t>(vnew + n16 * CH);
   }
   // Put the new token's rows in the place of row r (r % 16 of the step) of R.
   // Selects, not branches: a store to R under a condition on its index would
   // put R into scratch memory.
   __device__ __forceinline__ void patch_row(int r, const NewRow &nr, Regs &R) const {
-    if constexpr (!KT) {
-#pragma unroll
-      for (int i = 0; i < NQK; ++i) R.k[i] = n16 == (r & 15) ? nr.k[i] : R.k[i];
-    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const bool here = 4 * j + i == (r & 15);
-      if constexpr (KT) R.k[i] = here ? nr.k[0] : R.k[i];
+      R.k[i] = here ? nr.k : R.k[i];
       R.v[i] = here ? nr.v : R.v[i];
     }
   }
   // Write them at byte offset row_off of the pools (as row r).
   __device__ __forceinline__ void store_new(const char *kbase, const char *vbase, int64_t row_off,
                                             int r, const NewRow &nr) const {
-    char *kd = const_cast<char *>(kbase) + row_off, *vd = const_cast<char *>(vbase) + row_off;
-    if constexpr (!KT) {
-      if (n16 == (r & 15)) {
-#pragma unroll
-        for (int i = 0; i < NQK; ++i) store_vec<u32x4>(kd + (32 * i + 8 * j) * EB, nr.k[i]);
-      }
-    }
     if (j == (r & 15) >> 2) {
-      if constexpr (KT) store_vec<u32x4>(kd + n16 * CH * EB, nr.k[0]);
-      store_vec<vchunk_t>(vd + n16 * CH * EB, nr.v);
+      store_vec<u32x4>(const_cast<char *>(kbase) + row_off + n16 * CH * EB, nr.k);
+      store_vec<vchunk_t>(const_cast<char *>(vbase) + row_off + n16 * CH * EB, nr.v);
     }
   }
 
@@ -499,38 +484,6 @@ struct DecodeWaveF32 {
   }
 
   __device__ __forceinline__ void set_k_lds(char *) {}
-
-  // As DecodeWave's, with this wave's loads.
-  struct NewRow {
-    u32x4 k[NQK], v[VW];
-  };
-  __device__ __forceinline__ void load_new(const float *knew, const float *vnew,
-                                           NewRow &nr) const {
-#pragma unroll
-    for (int i = 0; i < NQK; ++i) nr.k[i] = load_vec<u32x4>(knew + 16 * i + 4 * j);
-#pragma unroll
-    for (int w = 0; w < VW; ++w) nr.v[w] = load_vec<u32x4>(vnew + 64 * w + 4 * n16);
-  }
-  __device__ __forceinline__ void patch_row(int r, const NewRow &nr, Regs &R) const {
-#pragma unroll
-    for (int i = 0; i < NQK; ++i) R.k[i] = n16 == (r & 15) ? nr.k[i] : R.k[i];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int w = 0; w < VW; ++w) R.v[c][w] = 4 * j + c == (r & 15) ? nr.v[w] : R.v[c][w];
-  }
-  __device__ __forceinline__ void store_new(const char *kbase, const char *vbase, int64_t row_off,
-                                            int r, const NewRow &nr) const {
-    char *kd = const_cast<char *>(kbase) + row_off, *vd = const_cast<char *>(vbase) + row_off;
-    if (n16 == (r & 15)) {
-#pragma unroll
-      for (int i = 0; i < NQK; ++i) store_vec<u32x4>(kd + (16 * i + 4 * j) * EB, nr.k[i]);
-    }
-    if (j == (r & 15) >> 2) {
-#pragma unroll
-      for (int w = 0; w < VW; ++w) store_vec<u32x4>(vd + (64 * w + 4 * n16) * EB, nr.v[w]);
-    }
-  }
 
   // As DecodeWave::col_of, for this wave's column placement.
   __device__ __forceinline__ static int col_of(int n16, int m) {

@@ -151,7 +151,17 @@ __device__ int block_exclusive_scan(int *buf, int n, int *tmp) {
   return total;
 }
 
-// APPEND (UNI only): fused append, see below.
+// The new row's registers of a fused append (nothing without one).
+template <class WV, bool APPEND>
+struct AppendRow {
+  struct type {};
+};
+template <class WV>
+struct AppendRow<WV, true> {
+  typedef typename WV::NewRow type;
+};
+
+// APPEND (K-transpose path only): fused append, see below.
 // KV8 (K-transpose path only): fp8 pools, see DecodeWave.
 // PART: split-K partials (partition_size > 0). The unit of the split is a
 // partition of partition_size tokens instead of a 16-token step (no phantom
@@ -311,12 +321,13 @@ paged_decode_stream(const DecodeParams p, const int32_t *__restrict__ tables,
     // adds no round trip to the wave (written before the ring and loaded back,
     // it added as much as an append launch of its own). The loads are
     // unconditional: a branch around them would make the compiler wait for
-    // every load in flight.
-    typename WV::NewRow nr;
+    // every load in flight. Other sequences' new rows are not ordered against
+    // this kernel's loads: no sequence may attend to another's new position.
+    typename AppendRow<WV, APPEND>::type nr;
     bool append = false;
     int64_t new_off = 0;
     if constexpr (APPEND) {
-      static_assert(UNI, "the new row replaces one row of a step in one block");
+      static_assert(UNI && D == 128 && sizeof(T) == 2, "stream_appends_in_kernel");
       const int64_t src = (int64_t)s_ * p.new_stride_seq + (int64_t)kvh * p.new_stride_head;
       w.load_new((const T *)p.key_new + src, (const T *)p.value_new + src, nr);
       const int nblk = brow[(ctx - 1) >> p.block_shift];
@@ -538,13 +549,13 @@ hipError_t launch_stream_tdd(const DecodeParams &p, hipStream_t stream) {
                          p.seg_prefix);
       return hipGetLastError();
     }
-  }
-  if (p.append_new) {  // set only where stream_appends_in_kernel holds
-    if (p.block_shift < 4) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH, true>), grid, dim3(kThreads), 0,
-                       stream, p, p.block_tables, p.context_lens, p.ws_o, p.ws_m, p.ws_l,
-                       p.seg_prefix);
-    return hipGetLastError();
+    if (p.append_new) {  // set only where stream_appends_in_kernel holds
+      if (p.block_shift < 4) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH, true>), grid, dim3(kThreads), 0,
+                         stream, p, p.block_tables, p.context_lens, p.ws_o, p.ws_m, p.ws_l,
+                         p.seg_prefix);
+      return hipGetLastError();
+    }
   }
   if (p.block_shift >= 4)
     hipLaunchKernelGGL((paged_decode_stream<T, D, true, DEPTH>), grid, dim3(kThreads), 0, stream,
@@ -611,20 +622,22 @@ bool decode_stream_supported(DType dt, int head_dim, int block_size, int64_t num
 }
 
 bool stream_appends_in_kernel(DType dt, int head_dim, int block_size, int group) {
-  // A 16-token step inside one block, with one query-head chunk per kv head:
-  // then a single wave loads the appended row. Against an append launch of its
-  // own (fp32 and head_dim 64): 2 sequences of 1000..3000 tokens, 32/8 heads,
-  // fp32 23.9 -> 18.8 us a call (with the host's share), 16 of 500..1500, 12
-  // heads of 64, fp16 22.7 -> 19.7; 16 of 256..4096, 28/4 heads, fp32 33.8 ->
-  // 33.2, where the append ran beside the stream kernel's start.
-  return (dt == DType::F16 || dt == DType::BF16 || dt == DType::F32) &&
-         (head_dim == 64 || head_dim == 128) && block_size >= 16 && group <= 16;
+  // The 16-bit K-transpose path (a 16-token step inside one block, head_dim
+  // 128) with one query-head chunk per kv head: a single wave then loads the
+  // appended row. It attends its own sequence's new row from registers, so a
+  // sequence whose table also covers another's new position would read the
+  // pool's old row there. fp32 pools and head_dim 64 append in a launch of
+  // their own, after which every sequence sees every new row (with them in
+  // this kernel: 2 sequences of 1000..3000 tokens, 32/8 heads, fp32 18.8 us a
+  // call against 23.9; 16 of 256..4096, 28/4 heads, fp32 33.2 against 33.8).
+  return (dt == DType::F16 || dt == DType::BF16) && head_dim == 128 && block_size >= 16 &&
+         group <= 16;
 }
 
 hipError_t launch_decode_stream(const DecodeParams &p, DType dt, hipStream_t stream) {
   if (dt == DType::BF16) return launch_stream_t<__bf16>(p, stream);
   if (dt == DType::F16) return launch_stream_t<_Float16>(p, stream);
-  if (dt == DType::F32 && !p.kv_fp8) return launch_stream_t<float>(p, stream);
+  if (dt == DType::F32 && !p.kv_fp8 && !p.append_new) return launch_stream_t<float>(p, stream);
   return hipErrorInvalidValue;
 }
 

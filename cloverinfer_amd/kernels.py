@@ -530,7 +530,12 @@ def paged_attention_append(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
     batches whose contexts fit the single pass (at most 512 tokens, at most 16
     query heads per kv head, ``num_waves`` 0) are one single-pass launch,
     longer ones the balanced decode. Covers the shapes of the balanced decode
-    (:func:`append_fusable`), raises otherwise."""
+    (:func:`append_fusable`), raises otherwise.
+
+    Each sequence is only sure to see its own new row: no sequence's tokens
+    may include a position that another one of the call appends (a shared
+    prefix is fine). Batches that need it (several new tokens of one sequence
+    as rows) take :func:`reshape_and_cache` and then :func:`paged_attention`."""
     AppendDecodeLaunch(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                        max_context_len, key_new, value_new, scale, num_waves).launch()
 

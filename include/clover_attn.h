@@ -248,7 +248,16 @@ int clv_paged_decode_balanced_noalloc(const clv_decode_args *args, int32_t num_w
  * max_context_len <= 512 and at most 16 query heads per kv head (fp32, fp16
  * or bf16 pools, head_dim 64 or 128, block_size >= 4), the call is instead
  * one single-pass launch that appends and attends (as clv_paged_decode: no
- * merge; the workspace is not used). A sequence appends nothing when
+ * merge; the workspace is not used). In these two forms each sequence is only
+ * sure to see its own new row: the caller must see to it that no sequence's
+ * first context_lens[s] tokens include a position that another sequence of
+ * the call appends (sequences may share the blocks of a common prefix, not
+ * the block that one of them appends into, unless it lies past the others'
+ * contexts); entries that need that, such as several new tokens of one
+ * sequence as rows of one batch, take clv_reshape_and_cache and then the
+ * decode. In the other forms (fp32 pools or head_dim 64 past the single
+ * pass's range) the rows are written by a launch before the decode, and every
+ * sequence sees all of them. A sequence appends nothing when
  * context_lens[s] is outside [1, min(max_context_len,
  * max_blocks_per_seq*block_size)] or the slot's block-table entry is outside
  * [0, num_blocks). k_cache and v_cache are written. No counterpart kernel
