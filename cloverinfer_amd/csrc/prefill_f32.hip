@@ -186,7 +186,9 @@ chunked_prefill_f32(const PrefillArgs args) {
       }
     };
     // Lanes whose token is not readable (past the context, or in an unmapped
-    // block) read zeros from the buffer resource's range check.
+    // block) read zeros from the buffer resource's range check. The range is
+    // the bytes from a block's first row to the end of its last one, also
+    // where rows overlap.
     auto load_tile = [&](int tile) {
 #pragma unroll
       for (int i = 0; i < PASSES; ++i) {
@@ -195,7 +197,7 @@ chunked_prefill_f32(const PrefillArgs args) {
         const bool ok = bok && (int)t + (lrow - wrow) < kv_end;
         rvalid[i] = ok;
         const uint64_t boff = (uint64_t)(uint32_t)(bok ? rblk[i] : 0) * sblk32;
-        const int nrec = bok ? (int)(stok32 << p.block_shift) : 0;
+        const int nrec = bok ? (int)(stok32 * bmask) + D * 4 : 0;
         const uint32_t voff = ok ? (t & bmask) * stok32 + lane_off : 0x80000000u;
         kreg[i] = buf_load<u32x4>(make_rsrc_range(kbase + boff, nrec), voff);
         vreg[i] = buf_load<u32x4>(make_rsrc_range(vbase + boff, nrec), voff);

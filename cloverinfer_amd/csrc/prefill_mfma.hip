@@ -282,9 +282,10 @@ chunked_prefill_mfma(const PrefillArgs args) {
     }
   };
   // Rows are read through a buffer resource whose range is the rows of one
-  // block: a lane whose token is not readable (past the context, or in an
-  // unmapped block, which gets an empty range) reads zeros from the hardware
-  // range check, so there are no per-lane branches and no zero fills.
+  // block (to the end of its last row, also where rows overlap): a lane whose
+  // token is not readable (past the context, or in an unmapped block, which
+  // gets an empty range) reads zeros from the hardware range check, so there
+  // are no per-lane branches and no zero fills.
   auto load_tile = [&](int tile) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
@@ -293,7 +294,7 @@ chunked_prefill_mfma(const PrefillArgs args) {
       const bool ok = bok && (int)tok0 + (lrow - wrow) < kv_end;
       rvalid[i] = ok;
       const uint64_t boff = (uint64_t)(uint32_t)(bok ? rblk[i] : 0) * sblk32;
-      const int nrec = bok ? (int)(stok32 << kv.block_shift) : 0;
+      const int nrec = bok ? (int)(stok32 * bmask) + D * 2 : 0;
       const uint32_t voff = ok ? (tok0 & bmask) * stok32 + lane_off : 0x80000000u;
       kreg[i] = buf_load<u32x4>(make_rsrc_range(kv.kbase + boff, nrec), voff);
       vreg[i] = buf_load<u32x4>(make_rsrc_range(kv.vbase + boff, nrec), voff);

@@ -189,3 +189,33 @@ def test_prefill_max_query_len_none_and_too_small(dtype):
     assert_attention_close(got[:40], ref[:40], what="rows below max_query_len")
     assert torch.isnan(got[40:300]).all(), "rows at or past max_query_len must come out as NaN"
     assert_attention_close(got[300:], ref[300:], what="the second, shorter chunk")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("stride_token", ["zero", "overlapping", "head_major"])
+def test_prefill_pool_strides(dtype, stride_token):
+    """Pools whose token rows are one row (expanded), overlap, or lie head by
+    head: a view is read by its strides, whatever memory it shares."""
+    hq, hkv, d, bs = 4, 2, 64, 16
+    cached, new = [0, 70, 1500], [40, 9, 30]
+    print(f"pool strides {stride_token} {dtype}", flush=True)
+    q, k, v, tables, ctx, qsl = build(31, cached, new, hq, hkv, d, bs, dtype)
+    nb = k.shape[0]
+    g = torch.Generator().manual_seed(6)
+
+    def view():
+        if stride_token == "zero":
+            return torch.randn(nb, 1, hkv, d, generator=g).to(dtype).to(DEV).expand(nb, bs, hkv, d)
+        if stride_token == "overlapping":
+            flat = torch.randn(nb * hkv * 16 * d, generator=g).to(dtype).to(DEV)
+            return flat.as_strided((nb, bs, hkv, d), (hkv * 16 * d, 32, 16 * d, 1))
+        return torch.randn(nb, hkv, bs, d, generator=g).to(dtype).to(DEV).transpose(1, 2)
+
+    kg, vg = view(), view()
+    out = torch.full((q.shape[0], hq, d), float("nan"), dtype=dtype, device=DEV)
+    kernels.chunked_prefill(out, q.to(DEV), kg, vg, padded_tables(tables).to(DEV),
+                            torch.tensor(ctx, dtype=torch.int32, device=DEV),
+                            torch.tensor(qsl, dtype=torch.int32, device=DEV), max(new))
+    torch.cuda.synchronize()
+    ref = oracle_prefill(q, kg.cpu().contiguous(), vg.cpu().contiguous(), tables, ctx, qsl, d ** -0.5)
+    assert_attention_close(out.cpu(), ref, what=f"prefill, {stride_token} token rows")
