@@ -336,8 +336,9 @@ class AppendDecodeLaunch:
         a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                          max_context_len, scale)
         self.device = _require_device(q, key_new, value_new)
-        if not balanced_supported(a):
-            raise NotImplementedError("paged_attention_append covers the balanced decode's shapes only")
+        if not balanced_supported(a) or k_cache.dtype == FP8:
+            raise NotImplementedError("paged_attention_append covers the balanced decode's shapes "
+                                      "only, with fp32/fp16/bf16 pools")
         shape = (a.num_seqs, a.num_kv_heads, a.head_dim)
         if key_new.shape != shape or value_new.shape != shape:
             raise ValueError(f"key_new/value_new must be {shape}, got {tuple(key_new.shape)} and "
@@ -439,8 +440,9 @@ class SplitAppendDecode:
         a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                          max_context_len, scale)
         self.device = q.device
-        if not balanced_supported(a):
-            raise NotImplementedError("the split decode covers the balanced decode's shapes only")
+        if not balanced_supported(a) or k_cache.dtype == FP8:
+            raise NotImplementedError("the split decode covers the balanced decode's shapes only, "
+                                      "with fp32/fp16/bf16 pools")
         self.args = a
         self.num_waves = num_waves
         self.new_shape = (a.num_seqs, a.num_kv_heads, a.head_dim)
@@ -671,11 +673,8 @@ def _prefill_args(out, q, k_cache, v_cache, block_tables, context_lens, query_st
     num_blocks, bs, num_kv_heads, kd = k_cache.shape
     if kd != head_dim or num_heads % num_kv_heads:
         raise ValueError("q and the caches disagree on head_dim or the GQA grouping")
-    fp8 = k_cache.dtype == FP8
-    if out.dtype != q.dtype or (q.dtype != k_cache.dtype and not fp8):
-        raise ValueError("q, out and the caches must share one dtype")
-    if fp8 and q.dtype not in (torch.float16, torch.bfloat16):
-        raise ValueError("fp8 pools need float16 or bfloat16 queries")
+    if out.dtype != q.dtype or q.dtype != k_cache.dtype:
+        raise ValueError("q, out and the caches must share one dtype (fp8 pools are for decode)")
     if q.stride(2) != 1 or out.stride(2) != 1:
         raise ValueError("q and out need a contiguous head_dim")
     num_seqs = context_lens.shape[0]
@@ -721,7 +720,7 @@ def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     ``max_query_len`` must be at least every chunk length n_s (it sizes the
     launch; a row i >= max_query_len of its chunk comes out as NaN, in every
     kernel form); None computes it from ``query_start_loc`` with one small
-    device-to-host copy.
+    device-to-host copy. fp32/fp16/bf16 pools of the queries' dtype.
     """
     a = None
     if max_query_len is not None:

@@ -1,0 +1,39 @@
+"""Checks that the tensor-level entry points make on the host before anything
+is launched, on CPU tensors (with the device check alone taken out)."""
+import pytest
+import torch
+
+from cloverinfer_amd import kernels
+
+
+@pytest.fixture(autouse=True)
+def cpu_tensors(monkeypatch):
+    monkeypatch.setattr(kernels, "_require_device", lambda *t: t[0].device)
+
+
+def tensors(dtype, pool_dtype, n=3, hq=8, hkv=2, d=128, bs=16):
+    q = torch.zeros(n, hq, d, dtype=dtype)
+    k = torch.zeros(6, bs, hkv, d).to(pool_dtype)
+    bt = torch.zeros(n, 2, dtype=torch.int32)
+    cl = torch.ones(n, dtype=torch.int32)
+    return torch.empty_like(q), q, k, k.clone(), bt, cl
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_fp8_pools_only_where_a_kernel_reads_them(dtype):
+    """Calls whose kernels read 16- or 32-bit pools refuse fp8 ones: read as
+    16-bit elements they end past the pools."""
+    out, q, k, v, bt, cl = tensors(dtype, kernels.FP8)
+    qsl = torch.arange(4, dtype=torch.int32)
+    with pytest.raises(ValueError):
+        kernels.chunked_prefill(out, q, k, v, bt, cl, qsl, 1)
+    new = torch.zeros(3, 2, 128).to(kernels.FP8)
+    with pytest.raises(NotImplementedError):
+        kernels.paged_attention_append(out, q, k, v, bt, cl, 16, 32, new, new)
+    with pytest.raises(NotImplementedError):
+        kernels.SplitAppendDecode(out, q, k, v, bt, cl, 16, 32)
+    # a pool of the queries' dtype passes the same checks
+    out, q, k, v, bt, cl = tensors(dtype, dtype)
+    kernels._prefill_args(out, q, k, v, bt, cl, qsl, 1, None)
+    kernels.AppendDecodeLaunch(out, q, k, v, bt, cl, 16, 32, new.to(dtype), new.to(dtype))
+    kernels.SplitAppendDecode(out, q, k, v, bt, cl, 16, 32)
