@@ -717,7 +717,9 @@ int fill_prefill(const clv_prefill_args *a, clv::PrefillParams *out) {
   p.group = a->num_heads / a->num_kv_heads;
   p.block_shift = log2_int(a->block_size);
   p.max_blocks_per_seq = a->max_blocks_per_seq;
-  p.max_query_len = a->max_query_len;
+  // No chunk is longer than the rows there are: a loose bound then sizes no
+  // grid and overflows no tile count.
+  p.max_query_len = std::min(a->max_query_len, a->num_tokens);
   p.num_blocks = a->num_blocks;
   p.scale_log2 = a->scale * 1.4426950408889634f;
   p.cus_per_xcd = device_compute_units() / 8;

@@ -68,6 +68,9 @@ __device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {
 // Tiles up to which no item is long enough for a cut to pay.
 constexpr int kSplitMinTiles = 6;
 
+// Most items of a call (above, prefill_f32_supported sends it to the VALU form).
+constexpr int64_t kMaxItems = (int64_t)1 << 30;
+
 template <int D, bool SPLIT>
 __global__ void __launch_bounds__(kThreads, per_cu(D))
 chunked_prefill_f32(const PrefillArgs args) {
@@ -414,7 +417,7 @@ hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t
   args.bq = kRows / p.group;
   args.n_qtiles = max(1, (p.max_query_len + args.bq - 1) / args.bq);
   const int64_t total = (int64_t)p.num_seqs * p.num_kv_heads * args.n_qtiles;
-  if (total > (int64_t)1 << 30) return hipErrorInvalidValue;
+  if (total > kMaxItems) return hipErrorInvalidValue;
   if (sp != nullptr) {
     args.sp = *sp;
     hipLaunchKernelGGL((chunked_prefill_f32<D, true>), dim3((unsigned)sp->groups), dim3(kThreads),
@@ -434,11 +437,16 @@ hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t
 
 bool prefill_f32_supported(const PrefillParams &p, int block_size) {
   // One load instruction of a wave covers 256 / head_dim rows of one block,
-  // and offsets inside a block are 32-bit bytes.
+  // and offsets inside a block are 32-bit bytes. The grid of the unsplit form
+  // has a workgroup per (sequence, kv head, query tile).
   const uint64_t lim = (uint64_t)1 << 31;
-  return (p.head_dim == 64 || p.head_dim == 128) && block_size >= 4 && p.group <= kRows &&
-         (uint64_t)p.kv_stride_block * 4 < lim &&
-         ((uint64_t)p.kv_stride_token * 4 << p.block_shift) < lim;
+  if (!((p.head_dim == 64 || p.head_dim == 128) && block_size >= 4 && p.group <= kRows &&
+        (uint64_t)p.kv_stride_block * 4 < lim &&
+        ((uint64_t)p.kv_stride_token * 4 << p.block_shift) < lim))
+    return false;
+  const int64_t bq = kRows / p.group;
+  const int64_t n_q = std::max<int64_t>(1, (p.max_query_len + bq - 1) / bq);
+  return (int64_t)p.num_seqs * p.num_kv_heads * n_q <= kMaxItems;
 }
 
 PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p) {

@@ -166,7 +166,7 @@ def test_prefill_every_workgroup_takes_the_exact_pass():
     assert_attention_close(got, ref, what="prefill, exact pass in every workgroup")
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])  # MFMA and VALU kernels
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])  # the 16-bit and the fp32 kernel
 def test_prefill_max_query_len_none_and_too_small(dtype):
     """max_query_len=None is computed from query_start_loc; a value below the
     longest chunk makes that chunk's rows at or past it NaN (a loud error, not
@@ -219,3 +219,38 @@ def test_prefill_pool_strides(dtype, stride_token):
     torch.cuda.synchronize()
     ref = oracle_prefill(q, kg.cpu().contiguous(), vg.cpu().contiguous(), tables, ctx, qsl, d ** -0.5)
     assert_attention_close(out.cpu(), ref, what=f"prefill, {stride_token} token rows")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bound", [1 << 20, 2**31 - 1])
+def test_prefill_loose_max_query_len(dtype, bound):
+    """max_query_len is an upper bound, however loose: nothing of it sizes the
+    launch past the query rows there are."""
+    hq, hkv, d, bs = 12, 12, 64, 16
+    cached, new = [0, 70, 900], [300, 9, 30]
+    print(f"max_query_len {bound} {dtype}", flush=True)
+    q, k, v, tables, ctx, qsl = build(41, cached, new, hq, hkv, d, bs, dtype)
+    out = torch.full((q.shape[0], hq, d), float("nan"), dtype=dtype, device=DEV)
+    kernels.chunked_prefill(out, q.to(DEV), k.to(DEV), v.to(DEV), padded_tables(tables).to(DEV),
+                            torch.tensor(ctx, dtype=torch.int32, device=DEV),
+                            torch.tensor(qsl, dtype=torch.int32, device=DEV), bound)
+    torch.cuda.synchronize()
+    ref = oracle_prefill(q, k, v, tables, ctx, qsl, d ** -0.5)
+    assert_attention_close(out.cpu(), ref, what=f"max_query_len {bound}")
+
+
+def test_prefill_f32_more_tiles_than_a_grid():
+    """65535 one-token sequences of 64 heads under a loose max_query_len: more
+    (sequence, head, query tile) items than one grid may have."""
+    n, h, d, bs = 65535, 64, 64, 16
+    print("fp32 prefill, 65535 sequences", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(8)
+    q = torch.randn(n, h, d, generator=g, device=DEV)
+    k = torch.randn(4, bs, h, d, generator=g, device=DEV)
+    v = torch.randn(4, bs, h, d, generator=g, device=DEV)
+    bt = (torch.arange(n, dtype=torch.int32, device=DEV) % 4).view(n, 1)
+    out = torch.full_like(q, float("nan"))
+    kernels.chunked_prefill(out, q, k, v, bt, torch.ones(n, dtype=torch.int32, device=DEV),
+                            torch.arange(n + 1, dtype=torch.int32, device=DEV), 1 << 20)
+    torch.cuda.synchronize()
+    assert torch.equal(out, v[bt[:, 0].long(), 0])  # one token: its value row
