@@ -222,12 +222,36 @@ def load() -> ctypes.CDLL:
 _host = None
 _host_tried = False
 
+# What the native host code fills (host/call_args.cpp) and where: its
+# functions, and the layout they must have been compiled with.
+_FILLS = ("fill_decode_args", "fill_prefill_args", "fill_cache_args")
+
+
+def call_args_layout() -> tuple:
+    """ABI version, then size and the offsets of dtype and scale of each
+    argument block (the host module's ``call_args_layout``)."""
+    out = [ABI_VERSION]
+    for cls in (DecodeArgs, PrefillArgs, CacheArgs):
+        out += [ctypes.sizeof(cls), cls.dtype.offset]
+        out += [cls.scale.offset] if cls is not CacheArgs else []
+    return tuple(out)
+
+
+def _checked_host(mod):
+    """``mod`` without the functions that write argument blocks where it was
+    built for another layout of them (a module left from an older tree)."""
+    if getattr(mod, "call_args_layout", None) != call_args_layout():
+        for name in _FILLS:
+            setattr(mod, name, None)
+    return mod
+
 
 def load_host():
     """The Python layer's native host code (cloverinfer_amd/_lib/_clv_host.so,
     built by cloverinfer_amd/build.py), or None when it is absent or does not
     load: it is host plumbing, and the backend then stages payloads with
-    torch.stack and kernels.py fills argument blocks in Python."""
+    torch.stack and kernels.py fills argument blocks in Python (as it does
+    with a module that was built for another layout of them)."""
     global _host, _host_tried
     if _host_tried:
         return _host
@@ -243,7 +267,7 @@ def load_host():
                     spec = importlib.util.spec_from_file_location(_build.HOST_EXT_NAME, path)
                     mod = importlib.util.module_from_spec(spec)
                     spec.loader.exec_module(mod)
-                    _host = mod
+                    _host = _checked_host(mod)
                 except ImportError:
                     _host = None
             _host_tried = True

@@ -14,6 +14,7 @@
 #include <torch/extension.h>
 
 #include <cmath>
+#include <cstddef>
 #include <limits>
 
 namespace clv_host {
@@ -215,6 +216,13 @@ bool fill_cache_args(uintptr_t dst, py::object key_, py::object value_, py::obje
   a.num_blocks = (int32_t)k->size(0);
   *reinterpret_cast<clv_cache_args *>(dst) = a;
   return true;
+}
+
+py::tuple call_args_layout() {
+  return py::make_tuple(
+      (size_t)CLV_ABI_VERSION, sizeof(clv_decode_args), offsetof(clv_decode_args, dtype),
+      offsetof(clv_decode_args, scale), sizeof(clv_prefill_args), offsetof(clv_prefill_args, dtype),
+      offsetof(clv_prefill_args, scale), sizeof(clv_cache_args), offsetof(clv_cache_args, dtype));
 }
 
 }  // namespace clv_host

@@ -17,4 +17,8 @@ bool fill_prefill_args(uintptr_t dst, py::object out, py::object q, py::object k
 bool fill_cache_args(uintptr_t dst, py::object key, py::object value, py::object k, py::object v,
                      py::object slots);
 
+// What the blocks' layout was when this was compiled (cloverinfer_amd/_native.py,
+// call_args_layout): the functions above are called only where it still is.
+py::tuple call_args_layout();
+
 }  // namespace clv_host

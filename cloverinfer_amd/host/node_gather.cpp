@@ -158,4 +158,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("fill_decode_args", &clv_host::fill_decode_args, "clv_decode_args from tensors");
   m.def("fill_prefill_args", &clv_host::fill_prefill_args, "clv_prefill_args from tensors");
   m.def("fill_cache_args", &clv_host::fill_cache_args, "clv_cache_args from tensors");
+  m.attr("call_args_layout") = clv_host::call_args_layout();
 }

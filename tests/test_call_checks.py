@@ -1,9 +1,12 @@
 """Checks that the tensor-level entry points make on the host before anything
 is launched, on CPU tensors (with the device check alone taken out)."""
+import os
+import types
+
 import pytest
 import torch
 
-from cloverinfer_amd import kernels
+from cloverinfer_amd import _native, build, kernels
 
 
 @pytest.fixture(autouse=True)
@@ -37,3 +40,23 @@ def test_fp8_pools_only_where_a_kernel_reads_them(dtype):
     kernels._prefill_args(out, q, k, v, bt, cl, qsl, 1, None)
     kernels.AppendDecodeLaunch(out, q, k, v, bt, cl, 16, 32, new.to(dtype), new.to(dtype))
     kernels.SplitAppendDecode(out, q, k, v, bt, cl, 16, 32)
+
+
+def test_host_module_of_another_layout_fills_nothing():
+    """The native fills write whole argument blocks at an address: a module
+    compiled for another layout of them must not be called."""
+    if not os.path.exists(build.HOST_EXT_PATH):
+        build.build_host_ext()
+    host = _native.load_host()
+    assert host.call_args_layout == _native.call_args_layout()
+    assert all(callable(getattr(host, n)) for n in _native._FILLS)
+    wrong = list(host.call_args_layout)
+    for i in range(len(wrong) + 1):
+        layout = tuple(wrong[:i] + [wrong[i] + 8] + wrong[i + 1:]) if i < len(wrong) else None
+        mod = types.SimpleNamespace(gather_rows=host.gather_rows, call_args_layout=layout,
+                                    **{n: getattr(host, n) for n in _native._FILLS})
+        if layout is None:
+            del mod.call_args_layout  # built before there was one
+        mod = _native._checked_host(mod)
+        assert mod.gather_rows is host.gather_rows
+        assert all(getattr(mod, n) is None for n in _native._FILLS), layout

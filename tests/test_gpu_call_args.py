@@ -1,12 +1,21 @@
 """Argument blocks filled by the native host code against those the Python
 checks fill, byte for byte, and the calls it leaves to them."""
+import os
+
 import pytest
 import torch
 
-from cloverinfer_amd import _native, kernels
+from cloverinfer_amd import _native, build, kernels
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def host():
+    if not os.path.exists(build.HOST_EXT_PATH):
+        build.build_host_ext()
+    assert _native.load_host() is not None
 
 
 def tensors(dtype, fp8=False):
