@@ -732,11 +732,17 @@ def chunked_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     dev = q.device
     lib = _native.load()
     nbytes = lib.clv_prefill_workspace_bytes(a)
+    ws = None
     if nbytes:
         # From the caching allocator, on the launch's stream: its memory may be
-        # handed out again once this call's kernels are queued ahead.
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        # handed out again once this call's kernels are queued ahead. Where the
+        # device has no room left for it, the form that needs none runs.
+        try:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            pass
+    if ws is not None:
         _native.check(lib.clv_chunked_prefill_split(a, ws.data_ptr(), nbytes, _stream(dev)),
                       "clv_chunked_prefill_split")
-        return
-    _native.check(lib.clv_chunked_prefill(a, _stream(dev)), "clv_chunked_prefill")
+    else:
+        _native.check(lib.clv_chunked_prefill(a, _stream(dev)), "clv_chunked_prefill")

@@ -60,3 +60,26 @@ def test_host_module_of_another_layout_fills_nothing():
         mod = _native._checked_host(mod)
         assert mod.gather_rows is host.gather_rows
         assert all(getattr(mod, n) is None for n in _native._FILLS), layout
+
+
+@pytest.mark.parametrize("room", [True, False])
+def test_prefill_without_room_for_a_workspace(monkeypatch, room):
+    """A call that would be split needs no memory of its own to run: on a
+    device that is full it takes the form without a workspace."""
+    out, q, k, v, bt, cl = tensors(torch.float16, torch.float16)
+    calls = []
+    lib = types.SimpleNamespace(
+        clv_prefill_workspace_bytes=lambda a: 4096,
+        clv_chunked_prefill_split=lambda a, ws, n, s: calls.append(("split", n)) or 0,
+        clv_chunked_prefill=lambda a, s: calls.append(("whole",)) or 0)
+
+    def empty(*size, **kw):
+        if not room:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return torch.zeros(*size, **kw)
+
+    monkeypatch.setattr(kernels._native, "load", lambda: lib)
+    monkeypatch.setattr(kernels, "_stream", lambda dev: 0)
+    monkeypatch.setattr(torch, "empty", empty)
+    kernels.chunked_prefill(out, q, k, v, bt, cl, torch.arange(4, dtype=torch.int32), 1)
+    assert calls == ([("split", 4096)] if room else [("whole",)])
