@@ -336,14 +336,15 @@ class AppendDecodeLaunch:
         a = _decode_args(out, q, k_cache, v_cache, block_tables, context_lens, block_size,
                          max_context_len, scale)
         self.device = _require_device(q, key_new, value_new)
-        if not balanced_supported(a) or k_cache.dtype == FP8:
+        dtype = k_cache.dtype
+        if dtype == FP8 or not balanced_supported(a):
             raise NotImplementedError("paged_attention_append covers the balanced decode's shapes "
                                       "only, with fp32/fp16/bf16 pools")
         shape = (a.num_seqs, a.num_kv_heads, a.head_dim)
         if key_new.shape != shape or value_new.shape != shape:
             raise ValueError(f"key_new/value_new must be {shape}, got {tuple(key_new.shape)} and "
                              f"{tuple(value_new.shape)}")
-        if key_new.dtype != k_cache.dtype or value_new.dtype != k_cache.dtype:
+        if key_new.dtype != dtype or value_new.dtype != dtype:
             raise ValueError("key_new/value_new dtype must match the cache dtype")
         key_new, value_new = self._rows(key_new, value_new)
         self.args = a
