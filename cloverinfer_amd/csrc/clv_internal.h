@@ -122,6 +122,7 @@ struct PrefillArgs {
   PrefillSplit sp;         // split form only
   int32_t bq, n_qtiles;    // tokens per query tile, query tiles per sequence
   int32_t total;           // items (one workgroup per item)
+  int32_t xcd_run;         // fp32 unsplit form: items in a row on one XCD
 };
 
 // Most (sequence, query tile) pairs a split prefill keeps in LDS.

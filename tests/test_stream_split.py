@@ -8,7 +8,9 @@ host (no GPU call).
   weights; the merge finds each segment's partials through owner().
 * prefill_order_check.hip: the chunked prefill's dispatch order
   (dispatch_slot in csrc/prefill_mfma.hip) is a permutation that keeps every
-  work item in its round and dispatches later rounds heaviest tile first."""
+  work item in its round and dispatches later rounds heaviest tile first.
+* prefill_f32_order_check.hip: the fp32 prefill's (dealt_item in
+  csrc/prefill_f32.hip) is one that spreads a long chunk over the XCDs."""
 import os
 import shutil
 import subprocess
@@ -42,3 +44,7 @@ def test_stream_split_invariants():
 
 def test_prefill_dispatch_order():
     _run_host_check("prefill_order_check")
+
+
+def test_prefill_f32_dispatch_order():
+    _run_host_check("prefill_f32_order_check")
