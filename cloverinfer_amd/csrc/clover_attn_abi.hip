@@ -731,7 +731,7 @@ enum class PrefillKernel { kValu, kMfma, kF32 };
 
 PrefillKernel prefill_kernel(const clv::PrefillParams &p, DType dt, int block_size) {
   if (dt == DType::F32)
-    return clv::prefill_f32_supported(p, block_size) ? PrefillKernel::kF32 : PrefillKernel::kValu;
+    return clv::prefill_f32_chosen(p, block_size) ? PrefillKernel::kF32 : PrefillKernel::kValu;
   return clv::prefill_mfma_supported(dt, p.head_dim, block_size) ? PrefillKernel::kMfma
                                                                  : PrefillKernel::kValu;
 }

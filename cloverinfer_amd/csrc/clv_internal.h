@@ -162,7 +162,7 @@ hipError_t launch_reshape_and_cache_fp8(const CacheParams &p, int src_dtype, con
 PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &p);
 hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *sp,
                                hipStream_t stream);
-bool prefill_f32_supported(const PrefillParams &p, int block_size);
+bool prefill_f32_chosen(const PrefillParams &p, int block_size);
 PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p);
 hipError_t launch_prefill_f32(const PrefillParams &p, const PrefillSplit *sp, hipStream_t stream);
 hipError_t launch_prefill_valu(const PrefillParams &p, DType dt, hipStream_t stream);

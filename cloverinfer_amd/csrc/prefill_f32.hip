@@ -68,7 +68,7 @@ __device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {
 // Tiles up to which no item is long enough for a cut to pay.
 constexpr int kSplitMinTiles = 6;
 
-// Most items of a call (above, prefill_f32_supported sends it to the VALU form).
+// Most items of a call (above, prefill_f32_chosen sends it to the VALU form).
 constexpr int64_t kMaxItems = (int64_t)1 << 30;
 
 // Item of workgroup `block` in the unsplit form. Consecutive ids go round-robin
@@ -451,7 +451,35 @@ hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t
 
 }  // namespace
 
-bool prefill_f32_supported(const PrefillParams &p, int block_size) {
+// Calls of few rows per (sequence, kv head) that the VALU form does faster: a
+// workgroup of 64 rows spends its time on an item's start, and once the items
+// fill the device (`slots` workgroups) nothing hides it. Batches over ragged
+// contexts up to the given length, us of the MFMA form and of the VALU form:
+//   one token a sequence, not split:
+//     12/12 heads of 64: 64 x 190 17.8, 15.2; 1200 x 190 235, 153;
+//     32/32 of 128: 16 x 190 25.8, 23.7; 64 x 60 38.9, 16.9; 1200 x 60 619, 246;
+//     16/8 of 128: 64 x 190 26.5, 31.1; 128 x 190 47.6, 32.5;
+//     32/8 of 128: 64 x 190 27.8, 41.0; 128 x 60 22.9, 20.0; 512 x 60 76.2, 44.1;
+//     28/4 of 128: 512 x 60 42.8, 79.4;
+//   split:
+//     12/12 of 64: 128 x 500 58.8, 45.1; 128 x 1000 105, 124; 128 x 4000 288, 465;
+//     32/32 of 128: 16 x 500 45.9, 56.9; 64 x 500 165, 142;
+//     16/8 of 128: 128 x 500 81.5, 75.4; 32/8 of 128: 128 x 500 94.0, 127;
+//   every 32nd sequence brings 33 tokens:
+//     12/12 of 64: 64 x 190 (split) 37.7, 20.1; 1200 x 60 126, 95;
+//     16/8 of 128: 1200 x 190 632, 323;
+//   2.8 tokens a sequence on average: 12/12 of 64, 256 x 500 142, 150.
+static bool valu_is_faster(const PrefillParams &p, int64_t entries) {
+  const int64_t tokens = p.num_tokens, seqs = p.num_seqs, items = seqs * p.num_kv_heads;
+  const int64_t slots = per_cu(p.head_dim) * 8 * (int64_t)p.cus_per_xcd;
+  const int64_t tiles = (((int64_t)p.max_blocks_per_seq << p.block_shift) + kBK - 1) / kBK;
+  if (tiles <= kSplitMinTiles || entries > kPrefillSplitItems)
+    return p.group <= 4 && 2 * tokens <= 5 * seqs && items >= std::min(p.group, 2) * slots;
+  return tiles <= 16 && p.group <= 2 && tokens <= 2 * seqs &&
+         items >= (p.group * p.head_dim == 64 ? 1 : 2) * slots;
+}
+
+bool prefill_f32_chosen(const PrefillParams &p, int block_size) {
   // One load instruction of a wave covers 256 / head_dim rows of one block,
   // and offsets inside a block are 32-bit bytes. The grid of the unsplit form
   // has a workgroup per (sequence, kv head, query tile).
@@ -461,8 +489,9 @@ bool prefill_f32_supported(const PrefillParams &p, int block_size) {
         ((uint64_t)p.kv_stride_token * 4 << p.block_shift) < lim))
     return false;
   const int64_t bq = kRows / p.group;
-  const int64_t n_q = std::max<int64_t>(1, (p.max_query_len + bq - 1) / bq);
-  return (int64_t)p.num_seqs * p.num_kv_heads * n_q <= kMaxItems;
+  const int64_t entries =
+      p.num_seqs * std::max<int64_t>(1, ((int64_t)p.max_query_len + bq - 1) / bq);
+  return entries * p.num_kv_heads <= kMaxItems && !valu_is_faster(p, entries);
 }
 
 PrefillSplitShape prefill_f32_split_shape(const PrefillParams &p) {

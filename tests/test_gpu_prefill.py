@@ -254,3 +254,28 @@ def test_prefill_f32_more_tiles_than_a_grid():
                             torch.arange(n + 1, dtype=torch.int32, device=DEV), 1 << 20)
     torch.cuda.synchronize()
     assert torch.equal(out, v[bt[:, 0].long(), 0])  # one token: its value row
+
+
+@pytest.mark.parametrize("n,hi,long,hq,hkv,d", [
+    (64, 100, 1, 12, 12, 64), (63, 100, 1, 12, 12, 64),     # one round of items, up to six tiles
+    (64, 500, 1, 12, 12, 64), (63, 500, 1, 12, 12, 64),     # up to sixteen
+    (64, 540, 1, 12, 12, 64), (16, 190, 1, 32, 32, 128),    # past them; head_dim 128
+    (128, 190, 1, 16, 8, 128), (127, 190, 1, 16, 8, 128),   # two rounds, group 2
+    (130, 60, 196, 32, 8, 128), (130, 60, 197, 32, 8, 128),  # 2.5 tokens a sequence, group 4
+    (256, 60, 1, 28, 4, 128), (1025, 300, 1, 7, 1, 64),     # group 7
+    (1025, 300, 200, 8, 4, 64),                             # past the split's table
+])
+def test_prefill_f32_few_rows(n, hi, long, hq, hkv, d):
+    """Batches of one-token sequences in fp32, which run the VALU or the MFMA
+    form by their size, on both sides of the lines."""
+    print(f"few rows {n} x {hi} {hq}/{hkv} d={d}", flush=True)
+    g = torch.Generator().manual_seed(n + hi)
+    cached = torch.randint(0, hi, (n,), generator=g).tolist()
+    new = [1] * n
+    new[n // 3] = long
+    q, k, v, tables, ctx, qsl = build(n, cached, new, hq, hkv, d, 16, torch.float32)
+    got = run_prefill(q, k, v, tables, ctx, qsl, d ** -0.5)
+    ref = oracle_prefill(q, k, v, tables, ctx, qsl, d ** -0.5)
+    # fp32 sums of at most 700 terms: sqrt(700) * 2^-24 of unit-variance values
+    # and the scores' rounding stay under 1e-5.
+    assert_attention_close(got, ref, atol=1e-5, rtol=1e-5, what=f"few rows {n} x {hi}")
