@@ -5,7 +5,7 @@
 // throughout (v_mfma_f32_16x16x4f32, 256 FLOP per clock and CU, the bound of
 // this kernel).
 //
-// A workgroup (4 waves, two workgroups per CU) takes 64 query rows = bq
+// A workgroup (4 waves; two per CU, three at head_dim 64) takes 64 query rows = bq
 // tokens x G query heads of one kv head, 16 rows per wave, and streams
 // 32-token K/V tiles through a two-stage LDS ring; the global loads of tile
 // k + 1 are in flight while tile k is computed. 64 rows: a prompt of a few
@@ -19,7 +19,8 @@
 // over 2048 cached, 12 heads of 64, 1584 -> 192 us (76 TFLOP/s), 32/8 heads of
 // 128, 5069 -> 843 us (92 of the 154 TFLOP/s of a large fp32 product). The
 // matrix pipes are busy half the time: waves wait on each other's issue and
-// on LDS; short prompts are bound by the items' start and the merge.
+// on LDS; short prompts are bound by the items' start and the merge. Batches of
+// one-token rows stay with the VALU form (valu_is_faster).
 //
 // Fragments (lane = 16j + n16): the score MFMAs take K as A (row = token) and
 // Q as B (column = query row), so that the lane ends up with the scores of
@@ -65,7 +66,9 @@ __device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {
                                               __builtin_bit_cast(float, b), c, 0, 0, 0);
 }
 
-// Tiles up to which no item is long enough for a cut to pay.
+// Table width in tiles up to which a call is not split (measured as in
+// prefill_mfma.hip, sum of 24 to 28 batches' times unsplit and split): 4 tiles 491
+// and 586 us, 6 759 and 762, 7 933 and 800, 8 1200 and 981, 12 2065 and 1395.
 constexpr int kSplitMinTiles = 6;
 
 // Most items of a call (above, prefill_f32_chosen sends it to the VALU form).

@@ -121,7 +121,7 @@ __host__ __device__ inline int dispatch_slot(int i, int per_xcd, int valid, int 
 // 2 units for up to 128 rows and 4 for the start, 122.7 at 3 and 4, 116.7 at 3
 // and 8 (114.1 at 4 and 8, which loses 9 % where one-token rows are 90 % of 24
 // sequences: 59.1 against 64.6 us); 141.6 and 218 where tiles of up to 32 rows
-// are priced at 2 and 1.
+// are priced at 2 and 1. Swept with heads of 128 only; head_dim 64 takes the same.
 struct SplitCfg {
   static constexpr int kBK = clv::kBK;
   static constexpr int kItemUnits = 8;
@@ -131,7 +131,12 @@ struct SplitCfg {
   static __device__ __forceinline__ int snap(int share) { return max(8, share / 16); }
 };
 
-// Tiles up to which no item is long enough for a cut to pay.
+// Table width in tiles up to which a call is not split. 27 batches a width
+// (prompts, chunks over cached tokens, mixed steps, one-token rows; 28/4, 32/8 and
+// 32/32 heads of 128, 12/12 of 64), contexts as long as the table, sum of their
+// times unsplit and split: 8 tiles 681 and 831 us, 12 986 and 1004, 16 1270 and
+// 1191 (half of them slower split), 18 1481 and 1298, 24 2107 and 1689, 40 4231
+// and 2906. Above the line equal items that fill the device lose up to a fifth.
 constexpr int kSplitMinTiles = 16;
 
 template <typename T, int D, bool SPLIT>

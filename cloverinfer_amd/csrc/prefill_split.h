@@ -34,9 +34,15 @@ namespace clv {
 // The decision behind the split shapes: `rows` query rows per workgroup, `bk`
 // K/V tokens per tile, `per_cu` workgroups per compute unit, at most
 // `tile_units` units per tile; no split up to `min_tiles` tiles, nor (with
-// `even_rounds`) of equal chunks that fill whole rounds of the device.
+// `even_rounds`) of equal chunks whose items fill whole rounds of the device.
+//
+// It sees sizes, not lengths. What that costs: where a table is much wider than
+// the contexts, the schedule and an empty merge launch are 5 to 7 us of a call
+// that is not cut (28/4 heads, bf16, 512 blocks wide: a prompt of 100 tokens 12.3
+// and 18.6 us, one of 777 31.8 and 38.6), against what long contexts gain (one
+// row over 4000 tokens 104 -> 25, three chunks of 100 over 2000 70 -> 40).
 inline PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, int bk, int per_cu,
-                                      int tile_units, int min_tiles, bool even_rounds) {
+                                             int tile_units, int min_tiles, bool even_rounds) {
   const PrefillSplitShape none = {rows, 0};
   const int64_t bq = rows / p.group;
   const int64_t n_q = std::max<int64_t>(1, ((int64_t)p.max_query_len + bq - 1) / bq);
@@ -44,12 +50,19 @@ inline PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, i
   // The table width bounds every context: up to min_tiles tiles the longest
   // item is short, and the split would cost its merge launch.
   if (max_tiles <= min_tiles || p.cus_per_xcd <= 0) return none;
+  // Every sequence has an entry in LDS for each tile of the longest chunk, also
+  // those that bring less. Past the table (28/4 heads in 16 bits: 64 sequences
+  // with a chunk of over 576 tokens, 128 with one of over 288) the call runs
+  // unsplit, however uneven it is.
   const int64_t entries = (int64_t)p.num_seqs * n_q;
   if (entries > kPrefillSplitItems) return none;
   // Units are 32-bit on the device (an item's own are at most four tiles').
   if (entries * p.num_kv_heads * (max_tiles + 4) * tile_units >= (int64_t)1 << 30) return none;
-  // Chunks of one length that fill whole rounds of the device: the 16-bit
-  // kernel's natural order (dispatch_slot) makes them even already.
+  // Chunks of one length that fill whole rounds of the device: over equal cached
+  // lengths the 16-bit kernel's natural order (dispatch_slot) makes them even
+  // already (8 x 512 over 4096, 32/8 heads, 292 us, split 303). The lengths are not
+  // known here: over 0..8192 cached tokens the same chunks take 489 us unsplit and
+  // would take 364 split.
   const int groups = per_cu * p.cus_per_xcd * 8;
   if (even_rounds && (int64_t)p.num_tokens == (int64_t)p.num_seqs * p.max_query_len &&
       entries * p.num_kv_heads % groups == 0)
