@@ -157,8 +157,9 @@ hipError_t launch_append_by_table(const DecodeParams &p, int elem_bytes, hipStre
 // rounded to nearest even; key/value in CacheParams' elem_bytes (2 or 4).
 hipError_t launch_reshape_and_cache_fp8(const CacheParams &p, int src_dtype, const float *k_scales,
                                         const float *v_scales, hipStream_t stream);
-// fp16/bf16 prefill on MFMA, and fp32 prefill on MFMA; sp: the split's workspace, or null for one workgroup
-// per item.
+// fp16/bf16 prefill on MFMA, and fp32 prefill on MFMA; sp: the split's
+// workspace, or null for one workgroup per item. prefill_f32_chosen: whether
+// the fp32 kernel covers the call and is faster on it than the VALU form.
 PrefillSplitShape prefill_mfma_split_shape(const PrefillParams &p);
 hipError_t launch_prefill_mfma(const PrefillParams &p, DType dt, const PrefillSplit *sp,
                                hipStream_t stream);

@@ -57,8 +57,8 @@ struct SplitCfg {
   static constexpr int kItemUnits = 1;
   static constexpr int kMinShare = 3;
   static constexpr int kCutUnits = 3;
-  static __device__ __forceinline__ int tile_units(int) { return 1; }
-  static __device__ __forceinline__ int snap(int share) { return max(1, share / 16); }
+  static __host__ __device__ __forceinline__ int tile_units(int) { return 1; }
+  static __host__ __device__ __forceinline__ int snap(int share) { return max(1, share / 16); }
 };
 
 __device__ __forceinline__ f32x4 mfma(uint32_t a, uint32_t b, f32x4 c) {

@@ -127,8 +127,8 @@ struct SplitCfg {
   static constexpr int kItemUnits = 8;
   static constexpr int kMinShare = 16;
   static constexpr int kCutUnits = 40;
-  static __device__ __forceinline__ int tile_units(int rows) { return rows > 128 ? 4 : 3; }
-  static __device__ __forceinline__ int snap(int share) { return max(8, share / 16); }
+  static __host__ __device__ __forceinline__ int tile_units(int rows) { return rows > 128 ? 4 : 3; }
+  static __host__ __device__ __forceinline__ int snap(int share) { return max(8, share / 16); }
 };
 
 // Table width in tiles up to which a call is not split. 27 batches a width

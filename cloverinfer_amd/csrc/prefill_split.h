@@ -70,6 +70,23 @@ inline PrefillSplitShape prefill_split_shape(const PrefillParams &p, int rows, i
   return {rows, groups};
 }
 
+// Wave operations of the schedule. It also compiles for the host, where one
+// thread stands for the wave (tests/host/prefill_split_check.h).
+__host__ __device__ __forceinline__ int first_lane(int x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_readfirstlane(x);
+#else
+  return x;
+#endif
+}
+__host__ __device__ __forceinline__ bool is_first_lane() {
+#ifdef __HIP_DEVICE_COMPILE__
+  return (threadIdx.x & 63) == 0;
+#else
+  return true;
+#endif
+}
+
 // What a group left in the workspace: the item whose first part it holds
 // (rows 0: none; partial slot 2w + 1), and whether its first item was begun
 // by an earlier group (cont, partial slot 2w) and ends here. The item is
@@ -92,7 +109,8 @@ struct PrefillItem {
   int ctx, base_pos;     // cached tokens; position of row 0
   int kv_end;            // tokens the last row sees
 
-  __device__ __forceinline__ void set(const PrefillParams &p, int bq, int s_, int kvh_, int qt_) {
+  __host__ __device__ __forceinline__ void set(const PrefillParams &p, int bq, int s_, int kvh_,
+                                               int qt_) {
     s = s_;
     kvh = kvh_;
     qt = qt_;
@@ -118,14 +136,37 @@ struct PrefillSched {
   bool whole;      // nothing is cut: one item per group, one unit per item
 
   // Query tile at position pos of a sequence's nqs tiles.
-  static __device__ __forceinline__ int folded(int pos, int nqs) {
+  static __host__ __device__ __forceinline__ int folded(int pos, int nqs) {
     return (pos & 1) ? pos >> 1 : nqs - 1 - (pos >> 1);
   }
-  static __device__ __forceinline__ int tiles(int kv_end) {
+  static __host__ __device__ __forceinline__ int tiles(int kv_end) {
     return max(1, (kv_end + Cfg::kBK - 1) / Cfg::kBK);
   }
-  static __device__ __forceinline__ int seq_tiles(int n_new, int bq, int nq) {
+  static __host__ __device__ __forceinline__ int seq_tiles(int n_new, int bq, int nq) {
     return min(nq, (max(0, n_new) + bq - 1) / bq);
+  }
+
+  // Units of entry i (0: no tile there).
+  __host__ __device__ __forceinline__ int entry_units(const PrefillParams &p, int bq, int i) const {
+    const int s = i / nq, pos = i - s * nq;
+    PrefillItem it;
+    it.set(p, bq, s, 0, 0);
+    const int nqs = seq_tiles(it.n_new, bq, nq);
+    if (pos >= nqs) return 0;
+    it.set(p, bq, s, 0, folded(pos, nqs));
+    return Cfg::kItemUnits + tiles(it.kv_end) * Cfg::tile_units((it.q_hi - it.q0) * p.group);
+  }
+
+  // The rest of the schedule from one kv head's units, its items and the
+  // longest of them.
+  __host__ __device__ __forceinline__ void set_totals(int heads, int groups, int units, int items,
+                                                      int most) {
+    const int share = units * heads / min(groups, max(1, units * heads / Cfg::kMinShare));
+    whole = items * heads <= groups && most <= share + share / 4 + Cfg::kCutUnits;
+    C = first_lane(whole ? items : units);
+    N = C * heads;
+    W = whole ? max(1, N) : min(groups, max(1, N / Cfg::kMinShare));
+    tol = whole ? 0 : Cfg::snap(share);
   }
 
   // Fills buf (kPrefillSplitItems + 1 ints of LDS; tmp: 3 per wave) and the
@@ -141,18 +182,10 @@ struct PrefillSched {
     const int b = min(n, tid * per), e = min(n, b + per);
     int units = 0, count = 0, most = 0;
     for (int i = b; i < e; ++i) {
-      const int s = i / nq, pos = i - s * nq;
-      PrefillItem it;
-      it.set(p, bq, s, 0, 0);
-      const int nqs = seq_tiles(it.n_new, bq, nq);
-      int u = 0;
-      if (pos < nqs) {
-        it.set(p, bq, s, 0, folded(pos, nqs));
-        u = Cfg::kItemUnits + tiles(it.kv_end) * Cfg::tile_units((it.q_hi - it.q0) * p.group);
-        ++count;
-      }
+      const int u = entry_units(p, bq, i);
       buf[i] = u;
       units += u;
+      count += u > 0 ? 1 : 0;
       most = max(most, u);
     }
     // Inclusive scans over the wave, then over the waves' totals.
@@ -185,9 +218,7 @@ struct PrefillSched {
       tc += tmp[3 * w + 1];
       most = max(most, tmp[3 * w + 2]);
     }
-    const int H = p.num_kv_heads;
-    const int share = tu * H / min(groups, max(1, tu * H / Cfg::kMinShare));
-    whole = tc * H <= groups && most <= share + share / 4 + Cfg::kCutUnits;
+    set_totals(p.num_kv_heads, groups, tu, tc, most);
     int run = whole ? rc : ru;
     for (int i = b; i < e; ++i) {
       const int u = buf[i];
@@ -196,16 +227,12 @@ struct PrefillSched {
     }
     if (tid == 0) buf[n] = whole ? tc : tu;
     __syncthreads();
-    C = __builtin_amdgcn_readfirstlane(whole ? tc : tu);
-    N = C * H;
-    W = whole ? max(1, N) : min(groups, max(1, N / Cfg::kMinShare));
-    tol = whole ? 0 : Cfg::snap(share);
   }
 
   // Group of workgroup `block`, or -1. Consecutive ids go round-robin over the
   // 8 XCDs: each takes a contiguous run of the W groups in use (query tiles of
   // one kv head then share its L2), the idle workgroups spread over all of them.
-  __device__ __forceinline__ int group_of(int block) const {
+  __host__ __device__ __forceinline__ int group_of(int block) const {
     const int per_xcd = (W + 7) / 8;
     const int w = (block % 8) * per_xcd + block / 8;
     return block / 8 < per_xcd && w < W ? w : -1;
@@ -219,7 +246,8 @@ struct PrefillSched {
 
   // Entry holding unit rem of a kv head (0 <= rem < C): the last one with
   // pre[i] <= rem; 64 candidates a round, as in the decode's stream kernel.
-  __device__ __forceinline__ int find(int rem) const {
+  __host__ __device__ __forceinline__ int find(int rem) const {
+#ifdef __HIP_DEVICE_COMPILE__
     const int lane = threadIdx.x & 63;
     int lo = 0, len = n;
     while (len > 1) {
@@ -229,19 +257,22 @@ struct PrefillSched {
       lo += k * stride;
       len = min(stride, len - k * stride);
     }
-    return __builtin_amdgcn_readfirstlane(lo);
+    return first_lane(lo);
+#else
+    return (int)(std::upper_bound(pre, pre + n, rem) - pre) - 1;
+#endif
   }
 
   // First unit of group w. Never decreases in w: a bound only moves onto the
   // item border nearest to it.
-  __device__ __forceinline__ int bound(int w) const {
+  __host__ __device__ __forceinline__ int bound(int w) const {
     if (w <= 0) return 0;
     if (w >= W) return N;
     const int x = (int)((int64_t)w * N / W);
     const int kvh = x / C, rem = x - kvh * C;
     const int i = find(rem);
-    const int lo = __builtin_amdgcn_readfirstlane(pre[i]);
-    const int hi = __builtin_amdgcn_readfirstlane(pre[i + 1]);
+    const int lo = first_lane(pre[i]);
+    const int hi = first_lane(pre[i + 1]);
     const int dl = rem - lo, dh = hi - rem;
     if (min(dl, dh) > tol) return x;
     return kvh * C + (dl <= dh ? lo : hi);
@@ -249,14 +280,14 @@ struct PrefillSched {
 
   // Writes the cursor of group w, kCursorInts ints of LDS that only this
   // wave uses.
-  __device__ __forceinline__ void start(int w, int *cur) const {
+  __host__ __device__ __forceinline__ void start(int w, int *cur) const {
     int x = 0, x_end = 0, entry = 0;
     if (N > 0 && w < W) {
       x = bound(w);
       x_end = bound(w + 1);
       if (x < x_end) entry = find(x % C);
     }
-    if ((threadIdx.x & 63) == 0) {
+    if (is_first_lane()) {
       cur[0] = x;
       cur[1] = x_end;
       cur[2] = entry;
@@ -268,23 +299,23 @@ struct PrefillSched {
   // Next piece of the group: tiles [t0, t1) of the nt tiles of item it (an
   // item of no tokens counts one); false when the group is done. The cursor
   // lives in LDS because the kernels' tile loops leave it no registers.
-  static __device__ __forceinline__ bool next(const PrefillParams &p, int bq, int nq,
-                                              const int *pre, int *cur, PrefillItem &it, int &t0,
-                                              int &t1, int &nt) {
-    int x = __builtin_amdgcn_readfirstlane(cur[0]);
-    const int x_end = __builtin_amdgcn_readfirstlane(cur[1]);
-    int entry = __builtin_amdgcn_readfirstlane(cur[2]);
-    const int C = __builtin_amdgcn_readfirstlane(cur[3]);
-    const bool whole = __builtin_amdgcn_readfirstlane(cur[4]) != 0;
+  static __host__ __device__ __forceinline__ bool next(const PrefillParams &p, int bq, int nq,
+                                                       const int *pre, int *cur, PrefillItem &it,
+                                                       int &t0, int &t1, int &nt) {
+    int x = first_lane(cur[0]);
+    const int x_end = first_lane(cur[1]);
+    int entry = first_lane(cur[2]);
+    const int C = first_lane(cur[3]);
+    const bool whole = first_lane(cur[4]) != 0;
     bool found = false;
     while (!found && x < x_end) {
       const int kvh = x / C;
       const int rem = x - kvh * C;
       if (rem == 0) entry = 0;  // a kv head's first item
-      while (__builtin_amdgcn_readfirstlane(pre[entry + 1]) <= rem) ++entry;
+      while (first_lane(pre[entry + 1]) <= rem) ++entry;
       const int s = entry / nq;
-      const int lo = kvh * C + __builtin_amdgcn_readfirstlane(pre[entry]);
-      const int hi = kvh * C + __builtin_amdgcn_readfirstlane(pre[entry + 1]);
+      const int lo = kvh * C + first_lane(pre[entry]);
+      const int hi = kvh * C + first_lane(pre[entry + 1]);
       const int n_new = p.query_start_loc[s + 1] - p.query_start_loc[s];
       it.set(p, bq, s, kvh, folded(entry - s * nq, seq_tiles(n_new, bq, nq)));
       nt = tiles(it.kv_end);
@@ -297,7 +328,7 @@ struct PrefillSched {
       ++entry;
       found = t0 < t1;
     }
-    if ((threadIdx.x & 63) == 0) {
+    if (is_first_lane()) {
       cur[0] = x;
       cur[2] = entry;
     }

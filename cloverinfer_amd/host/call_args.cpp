@@ -3,10 +3,10 @@
 // kernels.py checks a call's tensors and copies some twenty-five pointers,
 // sizes and strides into a ctypes structure. In Python that is most of the
 // host's share of a small call: a KV append of 16 rows took 10 us a call with
-// a kernel of 2 us. These functions make the same checks and fill the same structure in one call; they
-// return false where any check fails or an object is not a plain tensor, and
-// the Python code then does it all again and raises its own error (or takes
-// what this one does not).
+// a kernel of 2 us. These functions make the same checks and fill the same
+// structure in one call; they return false where any check fails or an object
+// is not a plain tensor, and the Python code then does it all again and raises
+// its own error (or takes what this one does not).
 #include "call_args.h"
 
 #include <clover_attn.h>

@@ -10,7 +10,10 @@ host (no GPU call).
   (dispatch_slot in csrc/prefill_mfma.hip) is a permutation that keeps every
   work item in its round and dispatches later rounds heaviest tile first.
 * prefill_f32_order_check.hip: the fp32 prefill's (dealt_item in
-  csrc/prefill_f32.hip) is one that spreads a long chunk over the XCDs."""
+  csrc/prefill_f32.hip) is one that spreads a long chunk over the XCDs.
+* prefill_split_{mfma,f32}_check.hip: the even split of a prefill
+  (PrefillSched in csrc/prefill_split.h): every tile taken once, and every
+  cut item's pieces where the merge looks for them."""
 import os
 import shutil
 import subprocess
@@ -48,3 +51,8 @@ def test_prefill_dispatch_order():
 
 def test_prefill_f32_dispatch_order():
     _run_host_check("prefill_f32_order_check")
+
+
+@pytest.mark.parametrize("kernel", ["mfma", "f32"])
+def test_prefill_split_invariants(kernel):
+    _run_host_check(f"prefill_split_{kernel}_check")
