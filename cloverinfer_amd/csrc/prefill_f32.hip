@@ -455,14 +455,17 @@ hipError_t launch_td(const PrefillParams &p, const PrefillSplit *sp, hipStream_t
 }  // namespace
 
 // Calls of few rows per (sequence, kv head) that the VALU form does faster: a
-// workgroup of 64 rows spends its time on an item's start, and once the items
-// fill the device (`slots` workgroups) nothing hides it. Batches over ragged
-// contexts up to the given length, us of the MFMA form and of the VALU form:
+// workgroup of 64 rows spends its time on an item's start, and on few tokens, or
+// once the items fill the device (`slots` workgroups), nothing hides it. Batches
+// over ragged contexts up to the given length, us of the MFMA form and of the
+// VALU form:
 //   one token a sequence, not split:
-//     12/12 heads of 64: 64 x 190 17.8, 15.2; 1200 x 190 235, 153;
-//     32/32 of 128: 16 x 190 25.8, 23.7; 64 x 60 38.9, 16.9; 1200 x 60 619, 246;
-//     16/8 of 128: 64 x 190 26.5, 31.1; 128 x 190 47.6, 32.5;
-//     32/8 of 128: 64 x 190 27.8, 41.0; 128 x 60 22.9, 20.0; 512 x 60 76.2, 44.1;
+//     12/12 heads of 64: 1 x 190 15.4, 9.3; 64 x 190 17.8, 15.2; 1200 x 190 235, 153;
+//     32/32 of 128: 4 x 100 17.4, 10.2; 64 x 60 38.9, 16.9; 1200 x 60 619, 246;
+//     16/8 of 128: 4 x 100 14.2, 12.5; 32 x 190 25.2, 28.4; 128 x 190 47.6, 32.5;
+//     24/12 of 64: 16 x 100 11.2, 9.2; 64 x 190 19.3, 20.1;
+//     32/8 of 128: 16 x 60 11.1, 13.8; 64 x 190 27.8, 41.0; 128 x 60 22.9, 20.0;
+//       512 x 60 76.2, 44.1;
 //     28/4 of 128: 512 x 60 42.8, 79.4;
 //   split:
 //     12/12 of 64: 128 x 500 58.8, 45.1; 128 x 1000 105, 124; 128 x 4000 288, 465;
@@ -477,7 +480,8 @@ static bool valu_is_faster(const PrefillParams &p, int64_t entries) {
   const int64_t slots = per_cu(p.head_dim) * 8 * (int64_t)p.cus_per_xcd;
   const int64_t tiles = (((int64_t)p.max_blocks_per_seq << p.block_shift) + kBK - 1) / kBK;
   if (tiles <= kSplitMinTiles || entries > kPrefillSplitItems)
-    return p.group <= 4 && 2 * tokens <= 5 * seqs && items >= std::min(p.group, 2) * slots;
+    return p.group <= 4 && 2 * tokens <= 5 * seqs &&
+           (p.group == 1 || (p.group == 2 && tiles <= 4) || items >= 2 * slots);
   return tiles <= 16 && p.group <= 2 && tokens <= 2 * seqs &&
          items >= (p.group * p.head_dim == 64 ? 1 : 2) * slots;
 }

@@ -257,10 +257,11 @@ def test_prefill_f32_more_tiles_than_a_grid():
 
 
 @pytest.mark.parametrize("n,hi,long,hq,hkv,d", [
-    (64, 100, 1, 12, 12, 64), (63, 100, 1, 12, 12, 64),     # one round of items, up to six tiles
-    (64, 500, 1, 12, 12, 64), (63, 500, 1, 12, 12, 64),     # up to sixteen
-    (64, 540, 1, 12, 12, 64), (16, 190, 1, 32, 32, 128),    # past them; head_dim 128
-    (128, 190, 1, 16, 8, 128), (127, 190, 1, 16, 8, 128),   # two rounds, group 2
+    (1, 30, 1, 12, 12, 64), (5, 190, 1, 32, 32, 128),       # group 1, up to six tiles
+    (64, 500, 1, 12, 12, 64), (63, 500, 1, 12, 12, 64),     # up to sixteen, one round of items
+    (64, 540, 1, 12, 12, 64),                               # past them
+    (9, 127, 1, 16, 8, 128), (9, 150, 1, 16, 8, 128),       # group 2, up to four tiles
+    (128, 190, 1, 16, 8, 128), (127, 190, 1, 16, 8, 128),   # two rounds
     (130, 60, 196, 32, 8, 128), (130, 60, 197, 32, 8, 128),  # 2.5 tokens a sequence, group 4
     (256, 60, 1, 28, 4, 128), (1025, 300, 1, 7, 1, 64),     # group 7
     (1025, 300, 200, 8, 4, 64),                             # past the split's table
